@@ -192,6 +192,30 @@ int UploadPlan(ehip_ctx* ctx, const ehip_geometry& g, Plan&& plan, const int32_t
   return EHIP_OK;
 }
 
+// Query rows per item of the bf16 block kernel (PrefillMfmaBf16) for the
+// geometry, 0 when it does not cover it.
+int BlockPrefillRows(const ehip_geometry& g) {
+  const int64_t stride = ehip::BlockStride(g);
+  const int64_t slab_bytes = g.slab_blocks > 0 && stride > 0 &&
+                                     g.slab_blocks <= INT64_MAX / stride / 2
+                                 ? g.slab_blocks * stride * 2
+                                 : INT64_MAX;
+  return ehip::PrefillRowsPerItem(g.kv_dtype, g.head_dim,
+                                  g.kv_heads > 0 ? g.heads / g.kv_heads : 0, g.block_size,
+                                  slab_bytes);
+}
+
+// How the step's chunks are taken: by the bf16 block kernel where it covers
+// the geometry, else by the fp32-class one, which multiplies planes of the
+// operands and costs more (rows = 0: chunks stay on the decode kernels).
+ehip::PrefillShape StepPrefillShape(const ehip_geometry& g) {
+  ehip::PrefillShape s;
+  s.rows = BlockPrefillRows(g);
+  if (s.rows > 0 || g.kv_heads < 1) return s;
+  return ehip::PrefillSplitShape(g.kv_dtype, g.head_dim, g.heads / g.kv_heads,
+                                 ehip::BlockStride(g));
+}
+
 // The decode-side parameters of the uploaded step (everything but the
 // fused-append rows).
 ehip::DecodeParams StepDecodeParams(ehip_ctx* ctx, const float* q, const void* k_slab,
@@ -206,11 +230,12 @@ int LaunchAttention(ehip_ctx* ctx, const float* q, const void* k_slab, const voi
       plan.prefill.size() > static_cast<size_t>(INT32_MAX))
     return SetError(ctx, EHIP_INVALID_ARGUMENT, "too many work items");
   if (!plan.prefill.empty()) {
+    const bool bf16 = BlockPrefillRows(g) > 0;  // the bf16 block kernel, else the split one
     const bool aligned = reinterpret_cast<uintptr_t>(q) % 16 == 0 &&
                          reinterpret_cast<uintptr_t>(k_slab) % 16 == 0 &&
                          reinterpret_cast<uintptr_t>(v_slab) % 16 == 0 &&
                          ehip::BlockStride(g) % 8 == 0;
-    if (!aligned)
+    if (bf16 && !aligned)
       return SetError(ctx, EHIP_INVALID_ARGUMENT,
                       "prefill chunks need 16-byte aligned q and slabs (ehip_malloc gives 256)");
     ehip::PrefillParams pp{};
@@ -226,16 +251,21 @@ int LaunchAttention(ehip_ctx* ctx, const float* q, const void* k_slab, const voi
                                    g.head_dim;
     pp.err = ctx->d_err;
     pp.block_stride = ehip::BlockStride(g);
+    pp.head_stride = ctx->head_stride;
     pp.slab_blocks = g.slab_blocks;
     pp.n_items = static_cast<int32_t>(plan.prefill.size());
+    pp.rows_per_item = StepPrefillShape(g).rows;
     pp.heads = g.heads;
     pp.kv_heads = g.kv_heads;
     pp.group = g.heads / g.kv_heads;
     pp.d = g.head_dim;
     pp.bs = g.block_size;
     pp.scale_log2 = g.scale * 1.4426950408889634f;
+    pp.k_scale = k_scale;
+    pp.v_scale = v_scale;
     hipError_t e = hipSuccess;
-    if (!ehip::LaunchPrefillMfma(pp, ctx->stream, &e))
+    if (!(bf16 ? ehip::LaunchPrefillMfma(pp, ctx->stream, &e)
+               : ehip::LaunchPrefillSplit(pp, g.kv_dtype, ctx->stream, &e)))
       return SetError(ctx, EHIP_INTERNAL, "prefill plan for a shape the kernel does not cover");
     EHIP_HIP(ctx, e);
   }
@@ -685,7 +715,8 @@ int ContiguousAttention(ehip_ctx* ctx, const float* d_q, const float* d_k, const
   const ehip_step_desc s{1, 0, &qlen, &l_dim, offsets, ids.data(), nullptr};
   Plan plan;
   std::string err;
-  if (int rc = ehip::BuildPlan(g, s, ctx->tune, &plan, &err, 0, /*head_major=*/true))
+  if (int rc = ehip::BuildPlan(g, s, ctx->tune, &plan, &err, StepPrefillShape(g),
+                               /*head_major=*/true))
     return SetError(ctx, rc, "%s", err.c_str());
   if (int rc = UploadPlan(ctx, g, std::move(plan), nullptr, l_dim * d)) return rc;
   return LaunchAttention(ctx, d_q, d_k, d_v, d_out);
@@ -885,27 +916,12 @@ int ehip_paged_decode_attention_batched_bf16(
 
 // ------------------------------------------------------------ step path --
 
-namespace {
-// Query rows per MFMA prefill item for the geometry (0: chunks stay on the
-// decode kernels).
-int StepPrefillRows(const ehip_geometry& g) {
-  const int64_t stride = ehip::BlockStride(g);
-  const int64_t slab_bytes = g.slab_blocks > 0 && stride > 0 &&
-                                     g.slab_blocks <= INT64_MAX / stride / 2
-                                 ? g.slab_blocks * stride * 2
-                                 : INT64_MAX;
-  return ehip::PrefillRowsPerItem(g.kv_dtype, g.head_dim,
-                                  g.kv_heads > 0 ? g.heads / g.kv_heads : 0, g.block_size,
-                                  slab_bytes);
-}
-}  // namespace
-
 int ehip_step_upload(ehip_ctx* ctx, const ehip_geometry* geom, const ehip_step_desc* step) {
   if (int rc = CheckCtx(ctx)) return rc;
   if (!geom || !step) return SetError(ctx, EHIP_INVALID_ARGUMENT, "null geometry or step");
   Plan plan;
   std::string err;
-  if (int rc = ehip::BuildPlan(*geom, *step, ctx->tune, &plan, &err, StepPrefillRows(*geom)))
+  if (int rc = ehip::BuildPlan(*geom, *step, ctx->tune, &plan, &err, StepPrefillShape(*geom)))
     return SetError(ctx, rc, "%s", err.c_str());
   return UploadPlan(ctx, *geom, std::move(plan), nullptr);
 }
@@ -1133,7 +1149,7 @@ int ehip_plan_prefill_items(const ehip_geometry* geom, const ehip_step_desc* ste
   Plan plan;
   std::string err;
   if (int rc = ehip::BuildPlan(*geom, *step, ehip::ReadTuning(), &plan, &err,
-                               StepPrefillRows(*geom)))
+                               StepPrefillShape(*geom)))
     return rc;
   *n = static_cast<int64_t>(plan.prefill.size());
   const int64_t m = std::min<int64_t>(cap, *n);

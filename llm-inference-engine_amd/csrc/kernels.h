@@ -88,7 +88,7 @@ struct QueueState {
 
 struct PrefillParams {
   const float* q;           // [rows, H, d]
-  const void* k_slab;       // bf16 slabs
+  const void* k_slab;
   const void* v_slab;
   float* out;               // [rows, H, d]
   const PrefillItem* items;
@@ -98,14 +98,18 @@ struct PrefillParams {
   float* part_ml;           // [partials, g, 2]
   int32_t* err;
   int64_t block_stride;
+  int64_t head_stride;      // elements between kv heads (PrefillSplitMfma; see DecodeParams)
   int64_t slab_blocks;
   int32_t n_items;
+  int32_t rows_per_item;    // chunk rows of a full item
   int32_t heads;
   int32_t kv_heads;
   int32_t group;
   int32_t d;
   int32_t bs;
   float scale_log2;
+  const float* k_scale;     // INT8/FP8 KV: per-(block, kv head) scales [slab_blocks, Hkv]
+  const float* v_scale;
 };
 
 // Causal prefill chunks on MFMA (bf16 K/V, d = 128, g in {4, 8}, bs >= 16):
@@ -116,6 +120,14 @@ bool LaunchPrefillMfma(const PrefillParams& p, hipStream_t stream, hipError_t* e
 // prefill kernel does not cover it (bf16 K/V, d = 128, g in {4, 8}, bs >= 16,
 // slabs below 4 GiB).
 int PrefillRowsPerItem(int kv_dtype, int d, int group, int bs, int64_t slab_bytes);
+
+// Causal prefill chunks at fp32-class precision (paged_prefill_split.hip): fp32,
+// bf16, INT8 or FP8 K/V, d 64 or 128, any g up to 64, every block size, blocks
+// less than 4 GiB apart. False (nothing launched) for other shapes.
+bool LaunchPrefillSplit(const PrefillParams& p, int kv_dtype, hipStream_t stream,
+                        hipError_t* err);
+// How that kernel takes a step's chunks; rows = 0 where it does not cover.
+PrefillShape PrefillSplitShape(int kv_dtype, int d, int group, int64_t block_stride);
 
 // Launch the decode kernel family for the given plan (one wavefront per work
 // item; picks the specialised (dtype, d, g) kernel or the generic one), then,

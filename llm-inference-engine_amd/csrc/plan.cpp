@@ -76,6 +76,10 @@ Tuning ReadTuning() {
   t.joint = flag("EHIP_NO_JOINT", '1');
   t.prefill = flag("EHIP_PREFILL", '0');
   if (const char* v = std::getenv("EHIP_PREFILL_SPLIT")) t.prefill_split = std::strtod(v, nullptr);
+  if (const char* v = std::getenv("EHIP_PREFILL_TILES")) {
+    const long x = std::strtol(v, nullptr, 10);
+    if (x > 0) t.prefill_tiles = static_cast<int32_t>(std::min<long>(x, 1 << 20));
+  }
   if (const char* v = std::getenv("EHIP_DECODE_KERNEL")) t.decode_valu = std::strcmp(v, "valu") == 0;
   if (const char* v = std::getenv("EHIP_DECODE_TILE")) t.decode_tile16 = std::strcmp(v, "16") == 0;
   if (const char* v = std::getenv("EHIP_DECODE_BUFS")) t.decode_bufs3 = std::strcmp(v, "3") == 0;
@@ -522,7 +526,8 @@ int BuildQ8Groups(const ehip_geometry& g, Plan* plan, std::string* err) {
 }  // namespace
 
 int BuildPlan(const ehip_geometry& g, const ehip_step_desc& s, const Tuning& tune, Plan* plan,
-              std::string* err, int prefill_rows, bool head_major) {
+              std::string* err, const PrefillShape& shape, bool head_major) {
+  const int prefill_rows = shape.rows;
   ehip_geometry checked = g;
   if (head_major) {
     if (g.block_stride != int64_t{g.block_size} * g.head_dim)
@@ -620,19 +625,19 @@ int BuildPlan(const ehip_geometry& g, const ehip_step_desc& s, const Tuning& tun
       }
       std::fill(skip.begin() + row_base[b], skip.begin() + row_base[b + 1], 1);
     }
-    // Key splits: a block with more than twice the per-workgroup share of
-    // the step's tiles is cut into splits of about that share, so the last
-    // query blocks of a long chunk do not walk all their keys alone
+    // Key splits: a block with more than shape.split times the per-workgroup
+    // share of the step's tiles is cut into splits of about that share, so
+    // the last query blocks of a long chunk do not walk all their keys alone.
     // Tuning::prefill_split: 0 keeps every block whole; a number x > 0
-    // splits blocks longer than x shares (default 2: on C3, x = 1 measured
-    // 58.9 us per layer against 45.7 us, as the extra partials and merge cost
-    // more than the shorter critical path saves; the C5 re-prefill is the
-    // same either way).
-    const double split_mult = tune.prefill_split;
+    // splits blocks longer than x shares. bf16 block kernel (2): on C3, x = 1
+    // measured 58.9 us per layer against 45.7 us, as the extra partials and
+    // merge cost more than the shorter critical path saves; the C5 re-prefill
+    // is the same either way.
+    const double split_mult = tune.prefill_split >= 0 ? tune.prefill_split : shape.split;
     const bool split_ok = split_mult > 0.0;
     const int64_t share = std::max<int64_t>(
-        kMinPrefillSplitTiles,
-        (total_tiles * g.kv_heads + kPrefillSlots - 1) / kPrefillSlots);
+        tune.prefill_tiles > 0 ? tune.prefill_tiles : shape.min_tiles,
+        (total_tiles * g.kv_heads + shape.slots - 1) / shape.slots);
     // Tiles per key split of a block. The split count a row records must be
     // the number of pieces actually cut: with the cap on splits, ceil(tiles /
     // per) can fall below the count asked for (e.g. 626 tiles asked in 64

@@ -43,7 +43,9 @@ struct Tuning {
                                // always / never (default: when items <= the item target)
   bool joint = true;           // EHIP_NO_JOINT=1: no joint items over shared prefixes
   bool prefill = true;         // EHIP_PREFILL=0: chunk rows stay on the decode kernels
-  double prefill_split = 2.0;  // EHIP_PREFILL_SPLIT: key-split threshold in shares (0: none)
+  double prefill_split = -1;   // EHIP_PREFILL_SPLIT: key-split threshold in shares (0: none;
+                               // default: the chunk kernel's own, PrefillShape)
+  int32_t prefill_tiles = 0;   // EHIP_PREFILL_TILES: least tiles of a key split (0: the kernel's)
   bool decode_valu = false;    // EHIP_DECODE_KERNEL=valu: all-VALU decode kernels
   bool decode_tile16 = false;  // EHIP_DECODE_TILE=16: one 16-key MFMA half per tile
   bool decode_bufs3 = false;   // EHIP_DECODE_BUFS=3: three tiles in registers
@@ -195,20 +197,29 @@ int32_t RowSplitTokens(const ehip_geometry& g, int32_t base, int32_t len);
 // single-sequence decode's partition), without building the plan.
 int32_t SingleRowSplitTokens(const ehip_geometry& g, int64_t length, const Tuning& tune);
 
+// How the step's chunk kernel takes its work: query rows per item (0: no
+// kernel, chunk rows stay on the decode kernels), workgroups resident at once,
+// the least tiles of a key split, and the shares of the step's tiles past
+// which a block is split.
+struct PrefillShape {
+  int rows = 0;
+  int32_t slots = 512;
+  int32_t min_tiles = 8;
+  double split = 2.0;
+};
+
 // Validates the step (lengths, CSR offsets, every table id and slot in range)
-// and builds the plan. Chunks of at least kMinPrefillRows rows go to the MFMA
-// prefill kernel when it covers the geometry (prefill_rows > 0: query rows
-// per prefill work item; Tuning::prefill = false keeps every row on the
-// decode kernels); their rows get nsplit = 0.
+// and builds the plan. Chunks of at least kMinPrefillRows rows go to the
+// matrix-core chunk kernel when one covers the geometry (shape.rows > 0;
+// Tuning::prefill = false keeps every row on the decode kernels); their rows
+// get nsplit = 0.
 constexpr int32_t kMinPrefillRows = 16;
 constexpr int32_t kPrefillTile = 32;       // keys per prefill tile
-constexpr int32_t kPrefillSlots = 512;     // workgroups resident at once (2 per CU)
-constexpr int32_t kMinPrefillSplitTiles = 8;
 // head_major: K/V are one contiguous [Hkv, L, d] cache read through an
 // identity table (block_stride = bs * d, kv heads L * d apart), so the slab
 // rule block_stride >= Hkv * bs * d does not apply.
 int BuildPlan(const ehip_geometry& g, const ehip_step_desc& s, const Tuning& tune, Plan* plan,
-              std::string* err, int prefill_rows = 0, bool head_major = false);
+              std::string* err, const PrefillShape& shape = {}, bool head_major = false);
 
 // Plan for one row reading a device-resident table (single-sequence paged
 // decode): one row of `length` keys, table offset 0.

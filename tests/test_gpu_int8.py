@@ -249,3 +249,30 @@ def test_int8_entry_points_reject_other_geometries(gctx, ehip_mod):
         assert getattr(gctx, f"step_attention_{fmt}")(buf, buf, buf, buf, buf, buf) == \
             E.INVALID_ARGUMENT
     buf.free()
+
+
+@pytest.mark.parametrize("fmt", FORMATS)
+@pytest.mark.parametrize("H,Hkv,d,bs", [(32, 8, 128, 16), (8, 2, 64, 64), (8, 8, 128, 32),
+                                        (16, 2, 64, 16)])
+@pytest.mark.parametrize("T,P", [(16, 0), (17, 33), (45, 700)])
+def test_scaled_chunks_match_the_decode_kernels(ehip_mod, orc, tctx, fmt, H, Hkv, d, bs, T, P):
+    """Causal chunks over INT8/FP8 K/V on the chunk kernel, at the edges of its
+    tiles and in key splits: within the fp32 bar of the reference over the
+    dequantised K/V and of the same step with its rows on the decode kernels."""
+    lens, qlens = [T + P, 90], [T, 1]
+    pool = sum((L + bs - 1) // bs for L in lens) + 3
+    outs = []
+    for flag in ("1", "0"):
+        rng = np.random.default_rng(T + P + d)
+        gctx = tctx(EHIP_PREFILL=flag)
+        tabs = make_tables(rng, lens, bs, pool)
+        run = ScaledRun(gctx, ehip_mod, H, Hkv, d, bs, pool, seed=5, fmt=fmt)
+        past = [max(P, 1), 89]
+        run.step(orc, tabs, past, past, rng, 1.0)
+        q, got, _ = run.step(orc, tabs, qlens, lens, rng, 1.0)
+        run.check_slabs()
+        ref = run.reference(orc, q, tabs, qlens, lens)
+        assert rel_norm(got, ref) <= 1e-4, rel_norm(got, ref)
+        outs.append(got)
+        run.free()
+    assert rel_norm(outs[0], outs[1]) <= 1e-4

@@ -1,0 +1,129 @@
+"""Causal chunks on the fp32-class chunk kernel (csrc/paged_prefill_split.hip):
+fp32 K/V and the bf16 shapes the bf16 block kernel does not cover, at the
+edges of its tiles (16-vector blocks, 32-key tiles, key splits), against the
+oracle's restatement of PrefillAttentionVarlenF32 and against the same step
+with every row on the decode kernels (EHIP_PREFILL=0).
+
+Bars: 1e-4 relative per output vector, the decode kernels' fp32 bar: the
+products left out of the plane splits are below 3 * 2^-24 of |q||k| (and
+|p||v|) per term, sums are fp32 over at most a few thousand terms, and the
+hardware exponential is within 2^-22 at these arguments, which together stay
+an order of magnitude under it."""
+from types import SimpleNamespace
+
+import numpy as np
+import pytest
+
+from gpu_util import rel_norm
+from paged_util import scale_for
+
+pytestmark = pytest.mark.gpu
+
+BAR = 1e-4
+
+
+def make_case(orc, bf16, H, Hkv, d, bs, chunks, seed):
+    """Chunks (T, P) plus one decode row over a shuffled pool; poison outside."""
+    rng = np.random.default_rng(seed)
+    qlens = [t for t, _ in chunks] + [1]
+    lens = [t + p for t, p in chunks] + [77]
+    need = [-(-n // bs) for n in lens]
+    pool = sum(need) + 3
+    perm = rng.permutation(pool).astype(np.int32)
+    tables, at = [], 0
+    for n in need:
+        tables.append(perm[at:at + n].copy())
+        at += n
+    k = np.full((pool, Hkv, bs, d), 1e30, np.float32)
+    v = np.full_like(k, 1e30)
+    ks, vs = [], []
+    for t, n in zip(tables, lens):
+        kk = rng.standard_normal((Hkv, n, d)).astype(np.float32)
+        vv = rng.standard_normal((Hkv, n, d)).astype(np.float32)
+        if bf16:
+            kk = orc.bf16_bits_to_f32(orc.to_bf16_bits(kk))
+            vv = orc.bf16_bits_to_f32(orc.to_bf16_bits(vv))
+        for s in range(n):
+            k[t[s // bs], :, s % bs] = kk[:, s]
+            v[t[s // bs], :, s % bs] = vv[:, s]
+        ks.append(kk)
+        vs.append(vv)
+    q = rng.standard_normal((sum(qlens), H, d)).astype(np.float32)
+    return SimpleNamespace(bf16=bf16, H=H, Hkv=Hkv, d=d, bs=bs, qlens=qlens, lens=lens,
+                           tables=tables, pool=pool, k=k, v=v, ks=ks, vs=vs, q=q)
+
+
+def run(ctx, ehip_mod, orc, c, shift=0):
+    """The step's outputs; shift moves every operand by that many bytes."""
+    def up(a):
+        b = ctx.alloc(a.nbytes + shift)
+        raw = np.zeros(a.nbytes + shift, np.uint8)
+        raw[shift:] = a.view(np.uint8).ravel()
+        b.upload(raw)
+        return b, SimpleNamespace(ptr=b.ptr + shift)
+
+    k = orc.to_bf16_bits(c.k) if c.bf16 else c.k
+    v = orc.to_bf16_bits(c.v) if c.bf16 else c.v
+    bufs = [up(a) for a in (c.q, k, v, np.zeros_like(c.q))]
+    dt = ehip_mod.KV_BF16 if c.bf16 else ehip_mod.KV_F32
+    g = ehip_mod.geometry(c.H, c.Hkv, c.d, c.bs, dt, c.pool, scale_for(c.d))
+    st = ehip_mod.StepArrays(c.qlens, c.lens, c.tables)
+    assert ctx.step_upload(g, st) == 0, ctx.last_error()
+    assert ctx.step_attention(*(p for _, p in bufs)) == 0, ctx.last_error()
+    ctx.sync()
+    raw = bufs[3][0].download(np.uint8, (c.q.nbytes + shift,))
+    for b, _ in bufs:
+        b.free()
+    return raw[shift:].view(np.float32).reshape(c.q.shape)
+
+
+def reference(orc, c):
+    cu = np.concatenate([[0], np.cumsum(c.qlens)]).astype(np.int32)
+    return orc.prefill_varlen(c.q, cu, c.ks, c.vs, c.H, c.Hkv, c.d, scale_for(c.d), isa=1)
+
+
+@pytest.mark.parametrize("bf16,H,Hkv,d,bs", [
+    (False, 14, 2, 64, 16), (False, 14, 2, 64, 8), (False, 8, 8, 64, 64), (False, 32, 8, 128, 16),
+    (False, 64, 1, 64, 16), (False, 6, 2, 128, 32), (True, 14, 2, 64, 16), (True, 8, 4, 128, 8),
+    (True, 32, 8, 128, 8)])
+@pytest.mark.parametrize("chunks", [[(16, 0), (17, 31)], [(33, 5), (130, 0)], [(40, 700)]],
+                         ids=["edges", "ragged", "splits"])
+def test_chunks_match_the_oracle(ehip_mod, orc, tctx, bf16, H, Hkv, d, bs, chunks):
+    c = make_case(orc, bf16, H, Hkv, d, bs, chunks, seed=H + d + bs + chunks[0][0])
+    ref = reference(orc, c)
+    ctx = tctx()
+    got = run(ctx, ehip_mod, orc, c)
+    assert rel_norm(got, ref) <= BAR, rel_norm(got, ref)
+    if chunks[0][1] == 700:  # 24 tiles: cut into key splits
+        assert ctx.step_info()[2] > 2 * Hkv
+    rows = run(tctx(EHIP_PREFILL="0"), ehip_mod, orc, c)
+    assert rel_norm(got, rows) <= BAR, rel_norm(got, rows)
+
+
+@pytest.mark.parametrize("bf16,d", [(False, 64), (False, 128), (True, 64)])
+def test_chunk_operands_at_any_alignment(gctx, ehip_mod, orc, bf16, d):
+    """q, slabs and outputs 4 bytes off a 16-byte boundary, as the decode
+    kernels take them (the decode row after the chunk takes another of them
+    there)."""
+    c = make_case(orc, bf16, 14, 2, d, 16, [(45, 20)], seed=d)
+    off, on = run(gctx, ehip_mod, orc, c, shift=4), run(gctx, ehip_mod, orc, c)
+    assert np.array_equal(off[:45], on[:45])
+    assert rel_norm(off, on) <= BAR
+
+
+@pytest.mark.parametrize("bf16,d", [(False, 64), (False, 128), (True, 64)])
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
+def test_rows_before_a_non_finite_value_stay_clean(gctx, ehip_mod, orc, bf16, d, bad):
+    """A non-finite V element reaches the rows that attend its key, in its
+    column, and no other output."""
+    c = make_case(orc, bf16, 14, 2, d, 16, [(70, 40)], seed=3 + d)
+    clean = run(gctx, ehip_mod, orc, c)
+    pos, col = 83, 9  # key 83 of the chunk's sequence: rows 43.. attend it
+    c.v[c.tables[0][pos // 16], 1, pos % 16, col] = bad
+    got = run(gctx, ehip_mod, orc, c)
+    hit = np.zeros(got.shape, bool)
+    hit[43:70, 7:, col] = True
+    assert rel_norm(got[~hit][None], clean[~hit][None]) <= BAR
+    assert not np.isfinite(got[hit]).any()
+    if not np.isnan(bad):
+        assert (got[hit] == (np.inf if bad > 0 else -np.inf)).all()
