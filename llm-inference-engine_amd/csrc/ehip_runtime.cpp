@@ -782,9 +782,7 @@ int ehip_packed_gemm(ehip_ctx* ctx, const float* d_x, int64_t m, int64_t k, cons
   {
     // x's bf16 planes, then (split k) the partial sums, 256 bytes apart.
     const size_t planes = (ehip::PackedGemmPlaneBytes(p) + 255) & ~size_t{255};
-    const size_t partial = p.splits > 1 ? static_cast<size_t>(p.splits) * static_cast<size_t>(m) *
-                                              static_cast<size_t>(n) * sizeof(float)
-                                        : 0;
+    const size_t partial = ehip::PackedGemmPartBytes(p);
     const size_t need = planes + partial;
     if (need > ctx->d_gemm_bytes) {
       const size_t bytes = std::max(need, ctx->d_gemm_bytes * 3 / 2);

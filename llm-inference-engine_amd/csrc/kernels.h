@@ -204,7 +204,8 @@ struct GemmParams {
   const void* wp;       // packed weight
   const float* bias;    // [n] or null
   float* y;             // [m, n]
-  float* part;          // [splits, m, n] partial sums (splits > 1)
+  float* part;          // partial sums (splits > 1): [splits, m, n], or with tile_rows > 0
+                        // [split tiles, splits, tile_rows, 256]
   int64_t m, k, n;
   int64_t m_pad, k_pad;  // m, k rounded up to whole 64 x 64 tiles
   int64_t panels;       // ceil(n / 16)
@@ -212,11 +213,22 @@ struct GemmParams {
   int64_t k_split;      // k per split (a multiple of 32)
   int32_t splits;
   int32_t x_vec;        // x rows are 16-byte aligned (k % 4 == 0, aligned base)
+  // The wide kernel (bf16 weights, k % 32 == 0): tiles of tile_rows x 256, the
+  // first full_tiles whole, the others in `splits` k ranges of split_steps
+  // 32-k steps; tile_rows = 0: the other kernel.
+  int32_t tile_rows;
+  int32_t row_tiles, col_tiles;
+  int32_t full_tiles;
+  int32_t split_steps;
+  int32_t items;        // workgroups
+  int32_t slots;        // workgroups resident at once
 };
 // Tiles and k splits for a call (cus: the device's CU count).
 void PlanPackedGemm(int64_t m, int64_t k, int64_t n, int weight_dtype, int cus, GemmParams* p);
 // Workspace bytes of x's planes for the planned call.
 size_t PackedGemmPlaneBytes(const GemmParams& p);
+// Workspace bytes of the planned call's partial sums.
+size_t PackedGemmPartBytes(const GemmParams& p);
 hipError_t LaunchPackedGemm(const GemmParams& p, int weight_dtype, hipStream_t stream);
 hipError_t LaunchPackWeightPanels(const void* w, int weight_dtype, int64_t n, int64_t k, void* wp,
                                   hipStream_t stream);

@@ -7,6 +7,9 @@
 // accumulation, and the bias added once after the k sum
 // (src/kernels/internal/gemm_common.h:22-41).
 //
+// Two kernels: PackedGemmWide for bf16 weights with k % 32 == 0 (below), and
+// PackedGemmMfma for the rest.
+//
 // Matrix-core form: every operand is cut into bf16 planes whose sum is the
 // value. x (fp32) takes three (x = x0 + x1 + x2, each the RNE bf16 of what the
 // earlier ones leave: about 2^-24 relative). Weights take as many as their
@@ -285,6 +288,262 @@ __global__ __launch_bounds__(kThreads) void PackedGemmMfma(GemmParams p) {
   }
 }
 
+// ------------------------------------------------------- bf16 weights, wide --
+//
+// The same product for bf16 weights with k % 32 == 0, as tiles of TM rows x 256
+// columns. What bounds the other kernel is the volume it moves from L2 to the
+// CUs (x's three planes per 64 x 128 or 64 x 256 tile: about 10 TB/s on a
+// 2382 x 4096 x 4096 call) and its pre-pass; here a workgroup of 8 wavefronts
+// covers up to 128 x 256, reads x as fp32 (two thirds of the planes' bytes) and
+// cuts it itself, 28 VALU instructions a thread per 32-k step under 48 MFMAs.
+//
+// Each 32-k step's x rows and panel rows are loaded two steps ahead into
+// registers, cut and stored in the LDS buffer the step before it is used: one
+// barrier a step. x planes sit in the A operand's own order (chunk q of a row
+// holds k 4q..4q+3 and 16+4q..+3), so an operand is one conflict-free 16-byte
+// read; panel rows sit as stored and are read transposed.
+//
+// Bound by the matrix cores' issue with two wavefronts a SIMD in step (MFMA busy
+// ~50% of a long call). Measured, this kernel against the other: 2382 x 4096 x
+// 4096 200 against 291 us a call, 256 x 4096 x 4096 35 against 51 us (28.6 + 7.4
+// us of split reduce), 32 x 896 x 896 9.3 against 21 us, 32 x 8192 x 8192 42
+// against 53 us. Interleaving the cuts with the MFMAs by scheduling groups took
+// the long call from 200 to 207 us.
+typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
+typedef __attribute__((ext_vector_type(2))) float f32x2_t;
+typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;
+
+constexpr int kWideN = 256;       // columns per tile (16 panels)
+constexpr int kWideK = 32;        // k per step
+constexpr int kWideThreads = 512;
+
+// Rows and columns of a wavefront: TM = 128 in 4 x 2 wavefronts of 32 x 128 (14
+// KB of operand reads per 48 MFMAs), fewer rows in more column groups.
+template <int TM>
+struct WideShape {
+  static constexpr int WR = TM >= 128 ? 4 : TM >= 64 ? 2 : 1;  // row groups
+  static constexpr int RB = TM / WR / 16;                      // 16-row blocks per wavefront
+  static constexpr int CB = kWideN / (8 / WR) / 16;            // panels per wavefront
+};
+
+template <int TM, int OCC>
+__global__ __launch_bounds__(kWideThreads) __attribute__((amdgpu_waves_per_eu(OCC)))
+void PackedGemmWide(GemmParams p) {
+  using S = WideShape<TM>;
+  constexpr int RB = S::RB, CB = S::CB;
+  __shared__ __align__(16) __bf16 xs[2][kXP][TM * kWideK];
+  __shared__ __align__(16) __bf16 ws[2][kWideN * kWideK];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = tid >> 6;
+  const int n16 = lane & 15;
+  const int q = lane >> 4;
+  const int wr = wave % S::WR;  // rows 16 RB wr .. of the tile
+  const int wc = wave / S::WR;  // panels CB wc .. of the tile
+
+  // Items: whole tiles first, then the last round's tiles in k splits. Tiles
+  // in bands of 4 row tiles, columns outer within a band, and an XCD (b mod 8)
+  // takes 32 consecutive ones a round: 4 x 8 tiles that share their x and
+  // panel rows in its L2. The splits of a tile are consecutive items, so with
+  // 8 of them an XCD keeps to one k range.
+  const int b = blockIdx.x;
+  int tile, split = 0, nsplit = 1;
+  if (b < p.full_tiles) {
+    const int round = b / p.slots, r = b - round * p.slots;
+    const int per = p.slots >> 3;
+    const bool whole = p.slots % 8 == 0 && (round + 1) * p.slots <= p.full_tiles;
+    tile = whole ? round * p.slots + (r & 7) * per + (r >> 3) : b;
+  } else {
+    nsplit = p.splits;
+    const int r = b - p.full_tiles;
+    tile = r / nsplit;
+    split = r - tile * nsplit;
+    tile += p.full_tiles;
+  }
+  const int band = tile / (4 * p.col_tiles);
+  const int in_band = tile - band * 4 * p.col_tiles;
+  const int h = min(4, p.row_tiles - 4 * band);
+  // Wavefront-uniform (readfirstlane): the divisions above leave vector
+  // registers, and buffer descriptors built from those would make every load a
+  // loop over its lanes' descriptors.
+  const int ct = __builtin_amdgcn_readfirstlane(in_band / h);
+  const int rt = __builtin_amdgcn_readfirstlane(4 * band + in_band - ct * h);
+  const int64_t m0 = int64_t{rt} * TM;
+  const int pb = ct * 16;
+  const int steps_all = static_cast<int>(p.k / kWideK);
+  const int s0 = __builtin_amdgcn_readfirstlane(nsplit > 1 ? split * p.split_steps : 0);
+  const int steps = nsplit > 1 ? min(p.split_steps, steps_all - s0) : steps_all;
+
+  // Loads: x row (tid / 4) mod TM, chunk tid % 4 (rows past m read the last
+  // one: their results are not stored); 16 bytes of panel wave + 8 i each.
+  const int xr = (tid >> 2) & (TM - 1);
+  const int64_t row_in = min(int64_t{xr}, p.m - 1 - m0);
+  const uint32_t xoff = static_cast<uint32_t>(row_in * p.k * 4) + (tid & 3) * 16;
+  const uint32_t pan0 = static_cast<uint32_t>(min(int64_t{wave}, p.panels - 1 - pb));
+  const uint32_t pan1 = static_cast<uint32_t>(min(int64_t{wave + 8}, p.panels - 1 - pb));
+  const uint32_t panel_b = static_cast<uint32_t>(p.k * kNr * 2);
+  const uint32_t woff0 = pan0 * panel_b + lane * 16;
+  const uint32_t woff1 = pan1 * panel_b + lane * 16;
+  const float* const xbase = p.x + m0 * p.k;
+  const uint16_t* const wbase = static_cast<const uint16_t*>(p.wp) + int64_t{pb} * p.k * kNr;
+  struct Stage {
+    u32x4_t x[2];
+    u32x4_t w[2];
+  };
+  // A step past the range reads nothing (empty buffers give zeros).
+  auto load = [&](int t, Stage& st) __attribute__((always_inline)) {
+    const uint32_t size = t < steps ? 0x7FFFFFFFu : 0u;
+    const __amdgpu_buffer_rsrc_t rx =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(xbase), 0, size, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rw =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(wbase), 0, size, 0x00020000);
+    const uint32_t xk = static_cast<uint32_t>(s0 + t) * (kWideK * 4);
+    const uint32_t wk = static_cast<uint32_t>(s0 + t) * (kWideK * kNr * 2);
+    st.x[0] = __builtin_amdgcn_raw_buffer_load_b128(rx, xoff, xk, 0);
+    st.x[1] = __builtin_amdgcn_raw_buffer_load_b128(rx, xoff + 64, xk, 0);
+    st.w[0] = __builtin_amdgcn_raw_buffer_load_b128(rw, woff0, wk, 0);
+    st.w[1] = __builtin_amdgcn_raw_buffer_load_b128(rw, woff1, wk, 0);
+  };
+  auto store = [&](const Stage& st, int buf) __attribute__((always_inline)) {
+    uint32_t pl[4][kXP];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float x = __uint_as_float(st.x[i >> 1][2 * (i & 1)]);
+      float y = __uint_as_float(st.x[i >> 1][2 * (i & 1) + 1]);
+#pragma unroll
+      for (int a = 0; a < kXP; ++a) {
+        const f32x2_t v = {x, y};
+        const bf16x2_t h = __builtin_convertvector(v, bf16x2_t);
+        pl[i][a] = __builtin_bit_cast(uint32_t, h);
+        if (a + 1 < kXP) {
+          x -= static_cast<float>(h[0]);
+          y -= static_cast<float>(h[1]);
+        }
+      }
+    }
+#pragma unroll
+    for (int a = 0; a < kXP; ++a)
+      *reinterpret_cast<u32x4_t*>(&xs[buf][a][xr * kWideK + (tid & 3) * 8]) =
+          u32x4_t{pl[0][a], pl[1][a], pl[2][a], pl[3][a]};
+    *reinterpret_cast<u32x4_t*>(&ws[buf][wave * 512 + lane * 8]) = st.w[0];
+    *reinterpret_cast<u32x4_t*>(&ws[buf][(wave + 8) * 512 + lane * 8]) = st.w[1];
+  };
+
+  f32x4_t acc[RB][CB];
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) acc[rb][cb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  auto compute = [&](int buf) __attribute__((always_inline)) {
+    bf16x8_t a[RB][kXP];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int pl = 0; pl < kXP; ++pl)
+        a[rb][pl] = *reinterpret_cast<const bf16x8_t*>(
+            &xs[buf][pl][(16 * (RB * wr + rb) + n16) * kWideK + q * 8]);
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) {
+      const __bf16* base =
+          &ws[buf][((CB * wc + cb) * kWideK + 4 * q + (n16 >> 2)) * kNr + 4 * (n16 & 3)];
+      const bf16x4_t lo = TransposedRead(base);
+      const bf16x4_t hi = TransposedRead(base + 16 * kNr);
+      const bf16x8_t w = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+      for (int pl = kXP - 1; pl >= 0; --pl)  // smallest plane first
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+          acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[rb][pl], w, acc[rb][cb], 0, 0, 0);
+    }
+  };
+  auto barrier = [&]() __attribute__((always_inline)) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  };
+
+  Stage st0, st1;
+  load(0, st0);
+  load(1, st1);
+  store(st0, 0);
+  load(2, st0);
+  barrier();
+  // Step t: store step t + 1, load step t + 3, compute step t. Past the range
+  // the stored planes and panel rows are zeros and add nothing.
+  for (int t = 0; t < steps; t += 2) {
+    store(st1, 1);
+    load(t + 3, st1);
+    compute(0);
+    barrier();
+    store(st0, 0);
+    load(t + 4, st0);
+    compute(1);
+    barrier();
+  }
+
+  // acc[rb][cb][i] = row 16 (RB wr + rb) + 4q + i, column n16 of panel CB wc + cb.
+  if (nsplit > 1) {
+    float* const part = p.part + (int64_t{tile - p.full_tiles} * nsplit + split) * (TM * kWideN);
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int row = 16 * (RB * wr + rb) + 4 * q + i;
+        if (m0 + row >= p.m) continue;
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb)
+          part[row * kWideN + (CB * wc + cb) * kNr + n16] = acc[rb][cb][i];
+      }
+    return;
+  }
+#pragma unroll
+  for (int cb = 0; cb < CB; ++cb) {
+    const int64_t col = int64_t{pb + CB * wc + cb} * kNr + n16;
+    if (col >= p.n) continue;
+    const float bias = p.bias ? p.bias[col] : 0.f;
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int64_t row = m0 + 16 * (RB * wr + rb) + 4 * q + i;
+        if (row < p.m) p.y[row * p.n + col] = acc[rb][cb][i] + bias;
+      }
+  }
+}
+
+// The split tiles: y = (partial 0 + partial 1 + ...) in split order, then +
+// bias; one thread per 4 columns of a tile row.
+__global__ __launch_bounds__(256) void WideSplitReduce(GemmParams p, int tm) {
+  const int quads = tm * (kWideN / 4);
+  const int e = static_cast<int>(blockIdx.y) * 256 + threadIdx.x;
+  if (e >= quads) return;
+  const int rt = static_cast<int>(blockIdx.x);
+  const int tile = rt + p.full_tiles;
+  const int band = tile / (4 * p.col_tiles);
+  const int in_band = tile - band * 4 * p.col_tiles;
+  const int h = min(4, p.row_tiles - 4 * band);
+  const int ct = in_band / h;
+  const int row = e / (kWideN / 4), c = (e - row * (kWideN / 4)) * 4;
+  const int64_t r = int64_t{4 * band + in_band - ct * h} * tm + row;
+  const int64_t col = int64_t{ct} * kWideN + c;
+  if (r >= p.m || col >= p.n) return;
+  const int64_t size = int64_t{tm} * kWideN;
+  const float* part = p.part + int64_t{rt} * p.splits * size + row * kWideN + c;
+  float4 s = *reinterpret_cast<const float4*>(part);
+  for (int i = 1; i < p.splits; ++i) {
+    const float4 v = *reinterpret_cast<const float4*>(part + i * size);
+    s.x += v.x;
+    s.y += v.y;
+    s.z += v.z;
+    s.w += v.w;
+  }
+  const float v[4] = {s.x, s.y, s.z, s.w};
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (col + i < p.n) p.y[r * p.n + col + i] = p.bias ? v[i] + p.bias[col + i] : v[i];
+}
+
 // x [m, k] fp32 -> its three bf16 planes [3][m_pad][k_pad], zero past m and
 // k; one thread per 8 consecutive elements of a padded row.
 __global__ __launch_bounds__(256) void SplitRows(GemmParams p, __bf16* xp) {
@@ -346,20 +605,72 @@ __global__ __launch_bounds__(256) void PackPanels(const T* w, int64_t n, int64_t
 
 }  // namespace
 
+namespace {
+
+// Row tile of the wide kernel for m rows: the one whose padded rows, with 32
+// rows' worth of panel staging per tile, come out smallest.
+int WideRows(int64_t m) {
+  int best = 128;
+  int64_t cost = INT64_MAX;
+  for (int tm : {128, 64, 32, 16}) {
+    const int64_t c = (m + tm - 1) / tm * (tm + 32);
+    if (c < cost) {
+      cost = c;
+      best = tm;
+    }
+  }
+  return best;
+}
+
+bool PlanWide(int64_t m, int64_t k, int64_t n, int cus, GemmParams* p) {
+  if (k % kWideK != 0 || k > (int64_t{1} << 21)) return false;  // whole steps, 32-bit offsets
+  const int tm = WideRows(m);
+  const int64_t rt = (m + tm - 1) / tm, ct = (p->panels + 15) / 16;
+  if (rt * ct > (int64_t{1} << 24)) return false;
+  const int steps = static_cast<int>(k / kWideK);
+  p->tile_rows = tm;
+  p->row_tiles = static_cast<int32_t>(rt);
+  p->col_tiles = static_cast<int32_t>(ct);
+  p->slots = cus * (tm <= 32 ? 2 : 1);
+  const int tiles = static_cast<int>(rt * ct);
+  p->full_tiles = tiles / p->slots * p->slots;
+  const int rem = tiles - p->full_tiles;
+  // The last round's tiles are cut over k so that it fills the chip: each
+  // split at least 4 steps, an even number of them (two per loop pass).
+  p->splits = 1;
+  p->split_steps = steps;
+  if (rem > 0) {
+    int s = p->slots / rem;
+    s = s > steps / 4 ? steps / 4 : s;
+    if (s > 1) {
+      const int per = ((steps + s - 1) / s + 1) / 2 * 2;
+      p->split_steps = per;
+      p->splits = (steps + per - 1) / per;
+    }
+  }
+  if (p->splits == 1) p->full_tiles = tiles;
+  p->items = p->full_tiles + (tiles - p->full_tiles) * p->splits;
+  return true;
+}
+
+}  // namespace
+
 void PlanPackedGemm(int64_t m, int64_t k, int64_t n, int weight_dtype, int cus, GemmParams* p) {
   // 16 panels (256 columns) per workgroup for bf16 weights and up to 256
   // rows: each x row is then staged for twice the columns (C4 o_proj 58.5 ->
   // 56 us, C5 63 -> 60 us). Taller calls keep 8 (C3's 2382 rows: 350 against
   // 365 us at 16), as do fp16 and fp32 weights, whose two or three weight
   // planes would not fit LDS at 16.
-  const int kBP = (weight_dtype == EHIP_WEIGHT_BF16 && m <= 256) ? 16 : 8;
-  p->group_panels = kBP;
   p->m = m;
   p->k = k;
   p->n = n;
+  p->panels = (n + kNr - 1) / kNr;
+  p->tile_rows = 0;
+  if (weight_dtype == EHIP_WEIGHT_BF16 && PlanWide(m, k, n, cus, p)) return;
+  const int kBP = (weight_dtype == EHIP_WEIGHT_BF16 && m <= 256) ? 16 : 8;
+  p->group_panels = kBP;
   p->m_pad = (m + kBM - 1) / kBM * kBM;
   p->k_pad = (k + kBK - 1) / kBK * kBK;
-  p->panels = (n + kNr - 1) / kNr;
   const int64_t tiles = ((m + kBM - 1) / kBM) * ((p->panels + kBP - 1) / kBP);
   const int64_t steps = (k + kBK - 1) / kBK;
   // Enough workgroups for one round at the tile's occupancy (two per CU for
@@ -377,12 +688,45 @@ void PlanPackedGemm(int64_t m, int64_t k, int64_t n, int weight_dtype, int cus, 
   p->splits = static_cast<int32_t>((steps + per - 1) / per);
 }
 
+size_t PackedGemmPartBytes(const GemmParams& p) {
+  if (p.splits <= 1) return 0;
+  if (p.tile_rows > 0)
+    return static_cast<size_t>(p.items - p.full_tiles) * p.tile_rows * kWideN * sizeof(float);
+  return static_cast<size_t>(p.splits) * static_cast<size_t>(p.m) * static_cast<size_t>(p.n) *
+         sizeof(float);
+}
+
 size_t PackedGemmPlaneBytes(const GemmParams& p) {
+  if (p.tile_rows > 0) return 0;  // the wide kernel cuts x itself
   return static_cast<size_t>(kXP) * static_cast<size_t>(p.m_pad) * static_cast<size_t>(p.k_pad) *
          sizeof(uint16_t);
 }
 
 hipError_t LaunchPackedGemm(const GemmParams& p, int weight_dtype, hipStream_t stream) {
+  if (p.tile_rows > 0) {
+    const dim3 grid(static_cast<uint32_t>(p.items)), block(kWideThreads);
+    switch (p.tile_rows) {
+      case 128:
+        hipLaunchKernelGGL((PackedGemmWide<128, 2>), grid, block, 0, stream, p);
+        break;
+      case 64:
+        hipLaunchKernelGGL((PackedGemmWide<64, 2>), grid, block, 0, stream, p);
+        break;
+      case 32:
+        hipLaunchKernelGGL((PackedGemmWide<32, 4>), grid, block, 0, stream, p);
+        break;
+      default:
+        hipLaunchKernelGGL((PackedGemmWide<16, 4>), grid, block, 0, stream, p);
+        break;
+    }
+    if (hipError_t e = hipGetLastError(); e != hipSuccess || p.splits == 1) return e;
+    const int tiles = (p.items - p.full_tiles) / p.splits;
+    hipLaunchKernelGGL(WideSplitReduce,
+                       dim3(static_cast<uint32_t>(tiles),
+                            static_cast<uint32_t>((p.tile_rows * (kWideN / 4) + 255) / 256)),
+                       dim3(256), 0, stream, p, static_cast<int>(p.tile_rows));
+    return hipGetLastError();
+  }
   {
     const int64_t groups = p.m_pad * (p.k_pad / 8);
     hipLaunchKernelGGL(SplitRows, dim3(static_cast<uint32_t>((groups + 255) / 256)), dim3(256), 0,

@@ -7,6 +7,8 @@ Bars: the device pack is bit-exact; the GEMM meets the reference's own GEMM
 tolerance (allclose rtol 1e-4, atol 1e-5 * sqrt(k), packed_gemm_test.cpp:180-184)
 over its shape list and the benchmark configurations' o_proj shapes; repeated
 calls are bit-identical (split-k partials added in split order)."""
+from types import SimpleNamespace
+
 import numpy as np
 import pytest
 
@@ -90,6 +92,38 @@ def test_packed_gemm_split_k_is_deterministic(gctx, ehip_mod, orc):
         dy.free()
     assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
     for b in (dw, dx, dwp):
+        b.free()
+
+
+@pytest.mark.parametrize("m,k,n", [
+    (1, 32, 16), (16, 96, 250), (17, 64, 256), (31, 128, 257), (33, 4096, 1111), (64, 160, 896),
+    (65, 896, 896), (127, 64, 4112), (128, 544, 272), (129, 256, 512), (257, 2048, 1000),
+    (2100, 64, 4096)])
+def test_wide_tiles_at_their_edges(gctx, ehip_mod, orc, m, k, n):
+    """bf16 weights with k % 32 == 0 (tiles of 16-128 rows x 256 columns): row
+    and column remainders, odd step counts, k splits of the last round's tiles
+    (the last shape has one whole round of them), and x and y 4 bytes off a
+    16-byte boundary. Bar: the reference's GEMM tolerance, against 64 bits."""
+    x = orc.fill_normal(m * k, 0.0, 1.0, m + k).reshape(m, k)
+    w = _weights(orc, ehip_mod, n, k, ehip_mod.WEIGHT_BF16, n + k)
+    bias = orc.fill_normal(n, 0.0, 1.0, 9)
+    dw, db = gctx.to_device(w), gctx.to_device(bias)
+    dwp = gctx.alloc(((n + 15) // 16) * k * 32)
+    assert gctx.pack_weight_panels(dw, ehip_mod.WEIGHT_BF16, n, k, dwp) == 0
+    raw = np.zeros(m * k + 1, np.float32)
+    raw[1:] = x.ravel()
+    dx, dy = gctx.to_device(raw), gctx.alloc(4 * (m * n + 2))
+    dy.upload(np.full(m * n + 2, 7.0, np.float32))
+    off = [SimpleNamespace(ptr=b.ptr + 4) for b in (dx, dy)]
+    assert gctx.packed_gemm(off[0], m, k, dwp, ehip_mod.WEIGHT_BF16, n, db, off[1]) == 0
+    gctx.sync()
+    out = dy.download(np.float32, (m * n + 2,))
+    assert out[0] == 7.0 and out[-1] == 7.0, "wrote outside y"
+    ref = x.astype(np.float64) @ orc.bf16_bits_to_f32(w).astype(np.float64).T + bias
+    err = np.abs(out[1:-1].reshape(m, n) - ref)
+    bad = err > 1e-5 * np.sqrt(k) + 1e-4 * np.abs(ref)
+    assert not bad.any(), (int(bad.sum()), float(err.max()))
+    for b in (dw, db, dwp, dx, dy):
         b.free()
 
 
