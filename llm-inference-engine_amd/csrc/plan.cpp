@@ -17,6 +17,12 @@ constexpr int32_t kTile = 64;             // split lengths are whole 64-key unit
 // first-tile round trips plus a partial slot, and the queue balances the
 // rest (with 32 item sub-queues, 2048 measured faster than 4096 on C3,
 // 150 -> 141 us, and C5, 268 -> 262 us; C4's items are all at the cap).
+// INT8/FP8 steps take the same target: with 1024, one wavefront a SIMD, the
+// VALU issue of their P.V starves (a wavefront alone issues an instruction
+// every ~8 cycles). Whole steps at 1024 / 2048 / 3072 items: FP8 mixed (60
+// decodes + chunks) 1333 / 1219 / 1226 us, 32 INT8 rows 567 / 531 / 561, 100
+// FP8 rows 1471 / 1295 / 1279, 12 INT8 rows of 8 heads a kv head 375 / 351 /
+// 414; 256 rows are at the length cap (7163 / 7144 / 7801).
 constexpr int64_t kTargetItems = 2048;
 constexpr int32_t kMinSplit = 128;
 // Steps this small (fewer than 128 items of kMinSplit keys) are latency-bound:
@@ -153,16 +159,16 @@ int32_t MaxSplitTokens(const ehip_geometry& g) {
   return 128 * g.block_size;
 }
 
-static int64_t DecodeItemTarget(const ehip_geometry& g, const Tuning& tune) {
+static int64_t DecodeItemTarget(const Tuning& tune) {
   if (tune.target_items > 0) return tune.target_items;
-  return ScaledKv(g.kv_dtype) ? kTargetItems / 2 : kTargetItems;
+  return kTargetItems;
 }
 
 int32_t ChooseSplitTokens(const ehip_geometry& g, int64_t unit_tokens, const Tuning& tune) {
   const int32_t max_split = MaxSplitTokens(g);
   if (tune.split_tokens > 0)
     return static_cast<int32_t>(std::min<int64_t>(RoundUp(tune.split_tokens, kTile), max_split));
-  const int64_t target = DecodeItemTarget(g, tune);
+  const int64_t target = DecodeItemTarget(tune);
   int64_t s = (unit_tokens + target - 1) / target;
   if (!ScaledKv(g.kv_dtype) && s >= kLargeStep) s = std::clamp(s, kLargeMin, kLargeMax);
   s = RoundUp(std::max<int64_t>(s, unit_tokens < kSmallStepUnits ? kTile : kMinSplit), kTile);
@@ -401,7 +407,7 @@ void FinishPlan(const ehip_geometry& g, const Tuning& tune, Plan* plan, bool all
   };
   cut_ranges(tune.split_even > 0);
   if (tune.split_even < 0 &&
-      static_cast<int64_t>(ranges.size()) * g.kv_heads <= DecodeItemTarget(g, tune))
+      static_cast<int64_t>(ranges.size()) * g.kv_heads <= DecodeItemTarget(tune))
     cut_ranges(true);
   CutTail(g, tune, plan->rows, &ranges);
 
