@@ -1043,8 +1043,9 @@ int ScaledAppend(ehip_ctx* ctx, int kv_dtype, const float* d_src_k, const float*
   if (ehip::BlockStride(g) != int64_t{g.kv_heads} * g.block_size * g.head_dim)
     return SetError(ctx, EHIP_UNIMPLEMENTED, "append needs the dense Hkv*bs*d block stride");
   EHIP_HIP(ctx, ehip::LaunchAppendQ8(d_src_k, d_src_v, ctx->d_q8_groups,
-                                     static_cast<int64_t>(plan.q8_groups.size()), ctx->d_q8_rows,
-                                     g.kv_heads, g.head_dim, g.block_size, g.slab_blocks,
+                                     static_cast<int64_t>(plan.q8_groups.size()),
+                                     plan.q8_max_rows, ctx->d_q8_rows, g.kv_heads, g.head_dim,
+                                     g.block_size, g.slab_blocks,
                                      d_k_slab, d_v_slab, d_k_scale, d_v_scale,
                                      kv_dtype == EHIP_KV_FP8, ctx->d_err, ctx->stream));
   return EHIP_OK;

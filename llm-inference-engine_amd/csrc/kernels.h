@@ -160,12 +160,13 @@ hipError_t LaunchKvGather(const float* k_slab, const float* v_slab, const int32_
                           int64_t slab_blocks, float* out_k, float* out_v, int32_t* err,
                           hipStream_t stream);
 
-// INT8 or FP8 (E4M3) append with per-(block, kv head) scales, one wavefront
-// per (append group, kv head).
+// INT8 or FP8 (E4M3) append with per-(block, kv head) scales, one workgroup per
+// (append group, kv head, K or V); max_rows: rows of the largest group.
 hipError_t LaunchAppendQ8(const float* src_k, const float* src_v, const Q8Group* groups,
-                          int64_t n_groups, const int32_t* rows, int kv_heads, int d, int bs,
-                          int64_t slab_blocks, void* k_slab, void* v_slab, float* k_scale,
-                          float* v_scale, bool fp8, int32_t* err, hipStream_t stream);
+                          int64_t n_groups, int max_rows, const int32_t* rows, int kv_heads,
+                          int d, int bs, int64_t slab_blocks, void* k_slab, void* v_slab,
+                          float* k_scale, float* v_scale, bool fp8, int32_t* err,
+                          hipStream_t stream);
 
 // Fused RoPE + KV append of one step's rows (q rotated in place; rotated K and
 // V scattered at the rows' slots; row r at position rows[r].length - 1).

@@ -203,9 +203,9 @@ __global__ __launch_bounds__(256) void RopeKvAppend(
   }
 }
 
-// INT8 / FP8 append with per-(block, kv head) scales. One wavefront per
-// (append group, kv head): the group's rows land at consecutive offsets
-// [off0, off0 + n) of one block. For K, then V: m = max |x| over the new rows;
+// INT8 / FP8 append with per-(block, kv head) scales. One workgroup per
+// (append group, kv head, K or V): the group's rows land at consecutive offsets
+// [off0, off0 + n) of one block. m = max |x| over the new rows;
 // the stored scale counts only when off0 > 0 (offset 0 is a freshly allocated
 // block, whatever an earlier owner left); if m exceeds R times that scale (R =
 // 127 for int8, 448 for E4M3), the scale becomes m / R and the block's older
@@ -213,8 +213,12 @@ __global__ __launch_bounds__(256) void RopeKvAppend(
 // of y = x * (1 / s): int8 clamp(rint(y), -127, 127); E4M3 of clamp(y, -448,
 // 448) rounded to nearest even (v_cvt_pk_fp8_f32 is exact RNE there), NaN
 // giving 0x7F. All in fp32 with round-to-nearest-even, so the slabs and
-// scales are bit-identical to the CPU restatement. Lanes handle 4 consecutive
-// elements (d % 4 == 0).
+// scales are bit-identical to the CPU restatement. Threads handle 4 consecutive
+// elements (d is 64 or 128) and keep the new rows' in registers between the
+// maximum and the codes. Bound by latency: one wavefront per block walked K then
+// V, each row's index, values and values again one after the other (20.6 us for
+// 3,048 chunk rows of 8 heads, d = 128); TPB = 256 spreads a filled block's rows
+// over four wavefronts and a decode step's single rows keep one.
 __device__ __forceinline__ int32_t Q8(float x, float inv, bool zero) {
   if (zero) return 0;
   const float y = fminf(fmaxf(rintf(x * inv), -127.0f), 127.0f);
@@ -264,55 +268,79 @@ __device__ __forceinline__ uint32_t Quant4(float4 x, float inv, bool zero) {
     return Pack4(Q8(x.x, inv, zero), Q8(x.y, inv, zero), Q8(x.z, inv, zero), Q8(x.w, inv, zero));
 }
 
-template <bool F8>
-__global__ __launch_bounds__(64) void AppendQ8(const float* __restrict__ src_k,
-                                               const float* __restrict__ src_v,
-                                               const Q8Group* __restrict__ groups,
-                                               const int32_t* __restrict__ rows, int kv_heads,
-                                               int d, int bs, int64_t slab_blocks,
-                                               uint8_t* k_slab, uint8_t* v_slab, float* k_scale,
-                                               float* v_scale, int32_t* err) {
+template <bool F8, int TPB>
+__global__ __launch_bounds__(TPB) void AppendQ8(const float* __restrict__ src_k,
+                                                const float* __restrict__ src_v,
+                                                const Q8Group* __restrict__ groups,
+                                                const int32_t* __restrict__ rows, int kv_heads,
+                                                int d, int bs, int64_t slab_blocks,
+                                                uint8_t* k_slab, uint8_t* v_slab, float* k_scale,
+                                                float* v_scale, int32_t* err) {
   constexpr float kRange = F8 ? 448.0f : 127.0f;
+  constexpr int kVecs = 8;  // float4 per thread: 64 rows of d = 128 over 256 threads
   const int gi = blockIdx.x / kv_heads;
   const int h = blockIdx.x - gi * kv_heads;
-  const int lane = threadIdx.x;
+  const int tid = threadIdx.x;
+  const bool v = blockIdx.y != 0;
   const Q8Group gr = groups[gi];
   if (gr.block < 0 || gr.block >= slab_blocks || gr.off0 < 0 || gr.off0 + gr.n > bs) {
-    if (lane == 0) atomicOr(err, kErrSlotRange);
+    if (tid == 0) atomicOr(err, kErrSlotRange);
     return;
   }
-  const int64_t tile = (int64_t{gr.block} * kv_heads + h) * bs * d;
-  const int d4 = d >> 2;
-  const int ne4 = gr.n * d4;
-  for (int which = 0; which < 2; ++which) {
-    const float* src = which ? src_v : src_k;
-    uint32_t* dst = reinterpret_cast<uint32_t*>((which ? v_slab : k_slab) + tile);
-    float* sc = (which ? v_scale : k_scale) + int64_t{gr.block} * kv_heads + h;
-    auto src4 = [&](int i) {
-      const int r = rows[gr.row0 + i / d4];
-      return *reinterpret_cast<const float4*>(src + (int64_t{r} * kv_heads + h) * d +
-                                              (i % d4) * 4);
-    };
-    float m = 0.f;
-    for (int i = lane; i < ne4; i += 64) {
-      const float4 x = src4(i);
-      m = fmaxf(m, fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w))));
+  const int sh = __builtin_ctz(d >> 2);  // float4 per row: 16 or 32
+  const int ne4 = gr.n << sh;
+  const float* const src = v ? src_v : src_k;
+  uint32_t* const dst = reinterpret_cast<uint32_t*>(
+      (v ? v_slab : k_slab) + (int64_t{gr.block} * kv_heads + h) * bs * d);
+  float* const sc = (v ? v_scale : k_scale) + int64_t{gr.block} * kv_heads + h;
+  const float s0 = gr.off0 > 0 ? *sc : 0.f;
+  float4 x[kVecs];
+  float m = 0.f;
+#pragma unroll
+  for (int j = 0; j < kVecs; ++j) {
+    const int i = tid + j * TPB;
+    x[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (i < ne4) {
+      const int r = rows[gr.row0 + (i >> sh)];
+      x[j] = *reinterpret_cast<const float4*>(src + (int64_t{r} * kv_heads + h) * d +
+                                              (i & ((1 << sh) - 1)) * 4);
     }
-    m = WaveMax(m);
-    const float s0 = gr.off0 > 0 ? *sc : 0.f;
-    float s1 = s0;
-    if (m > s0 * kRange) {
-      s1 = m / kRange;
-      const float inv = 1.0f / s1;
-      const bool zero = s1 == 0.0f;
-      for (int i = lane; i < gr.off0 * d4; i += 64)
-        dst[i] = Quant4<F8>(Unpack4<F8>(dst[i], s0), inv, zero);
-    }
+  }
+#pragma unroll
+  for (int j = 0; j < kVecs; ++j)
+    m = fmaxf(m, fmaxf(fmaxf(fabsf(x[j].x), fabsf(x[j].y)), fmaxf(fabsf(x[j].z), fabsf(x[j].w))));
+  m = WaveMax(m);
+  if constexpr (TPB > 64) {
+    __shared__ float wave_max[TPB / 64];
+    if ((tid & 63) == 0) wave_max[tid >> 6] = m;
+    __syncthreads();  // also: every thread has read the old scale
+    m = 0.f;
+#pragma unroll
+    for (int w = 0; w < TPB / 64; ++w) m = fmaxf(m, wave_max[w]);
+  }
+  float s1 = s0;
+  if (m > s0 * kRange) {
+    s1 = m / kRange;
     const float inv = 1.0f / s1;
     const bool zero = s1 == 0.0f;
-    for (int i = lane; i < ne4; i += 64) dst[gr.off0 * d4 + i] = Quant4<F8>(src4(i), inv, zero);
-    if (lane == 0) *sc = s1;
+    const int old4 = gr.off0 << sh;
+    for (int base = tid; base < old4; base += kVecs * TPB) {
+      uint32_t w[kVecs];
+#pragma unroll
+      for (int j = 0; j < kVecs; ++j) w[j] = base + j * TPB < old4 ? dst[base + j * TPB] : 0u;
+#pragma unroll
+      for (int j = 0; j < kVecs; ++j)
+        if (base + j * TPB < old4) dst[base + j * TPB] = Quant4<F8>(Unpack4<F8>(w[j], s0), inv, zero);
+    }
   }
+  const float inv = 1.0f / s1;
+  const bool zero = s1 == 0.0f;
+#pragma unroll
+  for (int j = 0; j < kVecs; ++j) {
+    const int i = tid + j * TPB;
+    if (i < ne4) dst[(gr.off0 << sh) + i] = Quant4<F8>(x[j], inv, zero);
+  }
+  if (tid == 0) *sc = s1;
 }
 
 // kernels::KvGatherF32 (src/kernels/kv_gather.cpp:42-89): out[h, j, :] is
@@ -372,16 +400,33 @@ int GridFor(int64_t work, int block) {
 }  // namespace
 
 hipError_t LaunchAppendQ8(const float* src_k, const float* src_v, const Q8Group* groups,
-                          int64_t n_groups, const int32_t* rows, int kv_heads, int d, int bs,
-                          int64_t slab_blocks, void* k_slab, void* v_slab, float* k_scale,
-                          float* v_scale, bool fp8, int32_t* err, hipStream_t stream) {
+                          int64_t n_groups, int max_rows, const int32_t* rows, int kv_heads,
+                          int d, int bs, int64_t slab_blocks, void* k_slab, void* v_slab,
+                          float* k_scale, float* v_scale, bool fp8, int32_t* err,
+                          hipStream_t stream) {
   if (n_groups <= 0) return hipSuccess;
-  if (d % 4 != 0 || n_groups * kv_heads > 0x7FFFFFFF) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(fp8 ? AppendQ8<true> : AppendQ8<false>,
-                     dim3(static_cast<uint32_t>(n_groups * kv_heads)), dim3(64), 0, stream,
-                     src_k, src_v, groups, rows, kv_heads, d, bs, slab_blocks,
-                     static_cast<uint8_t*>(k_slab), static_cast<uint8_t*>(v_slab), k_scale,
-                     v_scale, err);
+  if ((d != 64 && d != 128) || bs > 64 || n_groups * kv_heads > 0x7FFFFFFF)
+    return hipErrorInvalidValue;
+  // One wavefront while the largest group is two float4 a thread (four rows of
+  // d = 128), four past that.
+  const bool wide = max_rows * (d / 4) > 128;
+  const dim3 grid(static_cast<uint32_t>(n_groups * kv_heads), 2);
+#define EHIP_APPEND_Q8(F8, TPB)                                                                \
+  hipLaunchKernelGGL((AppendQ8<F8, TPB>), grid, dim3(TPB), 0, stream, src_k, src_v, groups,    \
+                     rows, kv_heads, d, bs, slab_blocks, static_cast<uint8_t*>(k_slab),        \
+                     static_cast<uint8_t*>(v_slab), k_scale, v_scale, err)
+  if (fp8) {
+    if (wide)
+      EHIP_APPEND_Q8(true, 256);
+    else
+      EHIP_APPEND_Q8(true, 64);
+  } else {
+    if (wide)
+      EHIP_APPEND_Q8(false, 256);
+    else
+      EHIP_APPEND_Q8(false, 64);
+  }
+#undef EHIP_APPEND_Q8
   return hipGetLastError();
 }
 

@@ -523,6 +523,7 @@ int BuildQ8Groups(const ehip_geometry& g, Plan* plan, std::string* err) {
     plan->q8_groups.push_back(Q8Group{static_cast<int32_t>(block), static_cast<int32_t>(off0),
                                       static_cast<int32_t>(j - i),
                                       static_cast<int32_t>(plan->q8_rows.size())});
+    plan->q8_max_rows = std::max(plan->q8_max_rows, static_cast<int32_t>(j - i));
     for (int64_t k = i; k < j; ++k) plan->q8_rows.push_back(order[k]);
     i = j;
   }
@@ -550,6 +551,7 @@ int BuildPlan(const ehip_geometry& g, const ehip_step_desc& s, const Tuning& tun
   plan->slots.clear();
   plan->q8_groups.clear();
   plan->q8_rows.clear();
+  plan->q8_max_rows = 0;
   plan->partials = 0;
   plan->max_length = 0;
   const int32_t B = s.num_seqs;

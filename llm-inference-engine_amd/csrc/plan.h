@@ -161,6 +161,7 @@ struct Plan {
   std::vector<int32_t> merge_rows;  // rows with more than one split, ascending
   std::vector<Q8Group> q8_groups;   // scaled-KV append groups (INT8/FP8 with slots)
   std::vector<int32_t> q8_rows;     // row indices of the groups, in offset order
+  int32_t q8_max_rows = 0;          // rows of the largest append group
   int64_t partials = 0;             // sum over rows of nsplit * Hkv
   int64_t max_length = 0;           // longest visible length (largest position + 1)
   int32_t split_tokens = 0;         // base split length chosen for this step
