@@ -57,6 +57,7 @@ struct ehip_ctx {
   const ehip::Q8Group* d_q8_groups = nullptr;  // INT8 append groups of the step
   const int32_t* d_q8_rows = nullptr;
   const int32_t* d_merge_rows = nullptr;
+  const ehip::SeqBase* d_seqs = nullptr;  // per-sequence caches of the uploaded call
   const ehip::ItemRowsX* d_items_x = nullptr;  // null unless the plan groups beyond pairs
 };
 
@@ -124,8 +125,10 @@ int UploadPlan(ehip_ctx* ctx, const ehip_geometry& g, Plan&& plan, const int32_t
   const size_t q8g_b = Align256(plan.q8_groups.size() * sizeof(ehip::Q8Group));
   const size_t q8r_b = Align256(plan.q8_rows.size() * sizeof(int32_t));
   const size_t itx_b = Align256(plan.items_x.size() * sizeof(ehip::ItemRowsX));
-  const size_t total = std::max<size_t>(
-      256, rows_b + items_b + prefill_b + table_b + slots_b + merge_b + q8g_b + q8r_b + itx_b);
+  const size_t seqs_b = Align256(plan.seqs.size() * sizeof(ehip::SeqBase));
+  const size_t total =
+      std::max<size_t>(256, rows_b + items_b + prefill_b + table_b + slots_b + merge_b + q8g_b +
+                                q8r_b + itx_b + seqs_b);
 
   const int cur = ctx->stage_cur;
   ctx->stage_cur ^= 1;
@@ -164,6 +167,8 @@ int UploadPlan(ehip_ctx* ctx, const ehip_geometry& g, Plan&& plan, const int32_t
   std::memcpy(h + q8_at + q8g_b, plan.q8_rows.data(), plan.q8_rows.size() * sizeof(int32_t));
   std::memcpy(h + q8_at + q8g_b + q8r_b, plan.items_x.data(),
               plan.items_x.size() * sizeof(ehip::ItemRowsX));
+  std::memcpy(h + q8_at + q8g_b + q8r_b + itx_b, plan.seqs.data(),
+              plan.seqs.size() * sizeof(ehip::SeqBase));
   EHIP_HIP(ctx, hipMemcpyAsync(ctx->d_desc, h, total, hipMemcpyHostToDevice, ctx->stream));
   if (!ctx->stage_done[cur]) EHIP_HIP(ctx, hipEventCreateWithFlags(&ctx->stage_done[cur],
                                                                    hipEventDisableTiming));
@@ -184,6 +189,9 @@ int UploadPlan(ehip_ctx* ctx, const ehip_geometry& g, Plan&& plan, const int32_t
   ctx->d_items_x = plan.items_x.empty()
                        ? nullptr
                        : reinterpret_cast<const ehip::ItemRowsX*>(d + q8_at + q8g_b + q8r_b);
+  ctx->d_seqs = plan.seqs.empty() ? nullptr
+                                  : reinterpret_cast<const ehip::SeqBase*>(
+                                        d + q8_at + q8g_b + q8r_b + itx_b);
   if (int rc = EnsureWorkspace(ctx, g, plan)) return rc;
   ctx->geom = g;
   ctx->plan = std::move(plan);
@@ -263,6 +271,7 @@ int LaunchAttention(ehip_ctx* ctx, const float* q, const void* k_slab, const voi
     pp.scale_log2 = g.scale * 1.4426950408889634f;
     pp.k_scale = k_scale;
     pp.v_scale = v_scale;
+    pp.seqs = ctx->d_seqs;
     hipError_t e = hipSuccess;
     if (!(bf16 ? ehip::LaunchPrefillMfma(pp, ctx->stream, &e)
                : ehip::LaunchPrefillSplit(pp, g.kv_dtype, ctx->stream, &e)))
@@ -801,6 +810,61 @@ int ehip_packed_gemm(ehip_ctx* ctx, const float* d_x, int64_t m, int64_t k, cons
   return EHIP_OK;
 }
 
+namespace {
+// Every member in one plan and launch of the fp32-class chunk kernel: its
+// items take their sequence's addresses from a table beside them, and its key
+// splits also serve short members (a decode-shaped one leaves most of its
+// vectors empty, but a plan, upload and launch of its own cost ~20 us: six
+// members of 1-400 rows over up to 1000 keys 118 -> 45 us a call). *done stays
+// false where the kernel does not cover the shape or the call exceeds one
+// plan's limits, and for one short member, which the decode kernels serve.
+int VarlenOneLaunch(ehip_ctx* ctx, const float* d_q, const int32_t* cu, int64_t num_seqs,
+                    const float* const* k_seqs, const float* const* v_seqs,
+                    const int64_t* l_dims, float* d_out, int64_t heads, int64_t kv_heads,
+                    int64_t d, float scale, bool* done) {
+  constexpr int32_t kRun = 16;
+  ehip::PrefillShape shape = ehip::PrefillSplitShape(
+      EHIP_KV_F32, static_cast<int>(d), static_cast<int>(heads / kv_heads), kRun * d);
+  if (shape.rows == 0 || !ctx->tune.prefill || cu[num_seqs] > (1 << 24) ||
+      (num_seqs == 1 && cu[1] < shape.min_rows))
+    return EHIP_OK;
+  shape.min_rows = 1;
+  int64_t blocks = 0, longest = 0;
+  for (int64_t b = 0; b < num_seqs; ++b) {
+    const int64_t n = (l_dims[b] + kRun - 1) / kRun;
+    blocks += n;
+    longest = std::max(longest, n);
+  }
+  if (blocks > INT32_MAX) return EHIP_OK;
+  std::vector<int32_t> qlens(num_seqs), offsets(num_seqs + 1, 0), ids;
+  ids.reserve(static_cast<size_t>(blocks));
+  std::vector<ehip::SeqBase> seqs(num_seqs);
+  for (int64_t b = 0; b < num_seqs; ++b) {
+    const int32_t n = static_cast<int32_t>((l_dims[b] + kRun - 1) / kRun);
+    qlens[b] = cu[b + 1] - cu[b];
+    offsets[b + 1] = offsets[b] + n;
+    for (int32_t i = 0; i < n; ++i) ids.push_back(i);
+    seqs[b] = ehip::SeqBase{reinterpret_cast<uint64_t>(k_seqs[b]),
+                            reinterpret_cast<uint64_t>(v_seqs[b]),
+                            l_dims[b] * d * static_cast<int64_t>(sizeof(float))};
+  }
+  const ehip_geometry g{static_cast<int32_t>(heads), static_cast<int32_t>(kv_heads),
+                        static_cast<int32_t>(d), kRun, EHIP_KV_F32, 0, longest, kRun * d, scale};
+  const ehip_step_desc s{static_cast<int32_t>(num_seqs), 0, qlens.data(), l_dims, offsets.data(),
+                         ids.data(), nullptr};
+  Plan plan;
+  std::string err;
+  if (int rc = ehip::BuildPlan(g, s, ctx->tune, &plan, &err, shape, /*head_major=*/true))
+    return SetError(ctx, rc, "%s", err.c_str());
+  plan.seqs = std::move(seqs);
+  if (int rc = UploadPlan(ctx, g, std::move(plan), nullptr)) return rc;
+  const int rc = LaunchAttention(ctx, d_q, k_seqs[0], v_seqs[0], d_out);
+  ctx->d_seqs = nullptr;  // the caller's addresses serve this call only
+  *done = true;
+  return rc;
+}
+}  // namespace
+
 int ehip_prefill_attention_varlen_f32(ehip_ctx* ctx, const float* d_q,
                                       const int32_t* h_cu_seqlens, int64_t num_seqs,
                                       const float* const* h_k_seqs,
@@ -834,6 +898,11 @@ int ehip_prefill_attention_varlen_f32(ehip_ctx* ctx, const float* d_q,
       return SetError(ctx, EHIP_INVALID_ARGUMENT, "sequence %lld: null K/V",
                       static_cast<long long>(b));
   }
+  bool launched = false;
+  if (int rc = VarlenOneLaunch(ctx, d_q, h_cu_seqlens, num_seqs, h_k_seqs, h_v_seqs, h_l_dims,
+                               d_out, heads, kv_heads, d, scale, &launched);
+      rc != EHIP_OK || launched)
+    return rc;
   const int64_t row = heads * d;
   for (int64_t b = 0; b < num_seqs; ++b) {
     const int64_t r0 = h_cu_seqlens[b];

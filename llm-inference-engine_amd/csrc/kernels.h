@@ -110,6 +110,7 @@ struct PrefillParams {
   float scale_log2;
   const float* k_scale;     // INT8/FP8 KV: per-(block, kv head) scales [slab_blocks, Hkv]
   const float* v_scale;
+  const SeqBase* seqs;      // per-sequence caches (PrefillSplitMfma over fp32), else null
 };
 
 // Causal prefill chunks on MFMA (bf16 K/V, d = 128, g in {4, 8}, bs >= 16):

@@ -201,9 +201,18 @@ void PrefillSplitMfma(PrefillParams p) {
   // multiply-add per loaded row; V sits at K's address plus a uniform distance.
   const uint32_t stride_b = static_cast<uint32_t>(p.block_stride * KT::ES);
   const uint32_t nblk = static_cast<uint32_t>(min(p.slab_blocks, int64_t{INT32_MAX}));
-  const int64_t head_off = int64_t{hk} * p.head_stride * KT::ES;
-  const uint64_t kbase = reinterpret_cast<uint64_t>(p.k_slab) + head_off;
-  const uint64_t v_from_k = reinterpret_cast<uint64_t>(p.v_slab) - reinterpret_cast<uint64_t>(p.k_slab);
+  uint64_t kbase = reinterpret_cast<uint64_t>(p.k_slab);
+  uint64_t v_from_k = reinterpret_cast<uint64_t>(p.v_slab) - kbase;
+  int64_t head_bytes = p.head_stride * KT::ES;
+  if constexpr (KV == EHIP_KV_F32) {
+    if (p.seqs != nullptr) {  // separate per-sequence caches
+      const SeqBase sb = p.seqs[it.seq];
+      kbase = sb.k;
+      v_from_k = sb.v - sb.k;
+      head_bytes = sb.head_bytes;
+    }
+  }
+  kbase += hk * head_bytes;
   const PairFactors pf = MakePairFactors();
   bool bad = false;
 

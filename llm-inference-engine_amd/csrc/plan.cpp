@@ -552,6 +552,7 @@ int BuildPlan(const ehip_geometry& g, const ehip_step_desc& s, const Tuning& tun
   plan->q8_groups.clear();
   plan->q8_rows.clear();
   plan->q8_max_rows = 0;
+  plan->seqs.clear();
   plan->partials = 0;
   plan->max_length = 0;
   const int32_t B = s.num_seqs;
@@ -625,7 +626,7 @@ int BuildPlan(const ehip_geometry& g, const ehip_step_desc& s, const Tuning& tun
     int64_t total_tiles = 0;
     for (int32_t b = 0; b < B; ++b) {
       const int32_t T = s.h_query_lens[b];
-      if (T < kMinPrefillRows) continue;
+      if (T < shape.min_rows) continue;
       const int32_t P = static_cast<int32_t>(s.h_context_lens[b] - T);
       for (int32_t q0 = 0; q0 < T; q0 += prefill_rows) {
         blocks.push_back({b, q0, P + std::min(T, q0 + prefill_rows)});
@@ -687,7 +688,7 @@ int BuildPlan(const ehip_geometry& g, const ehip_step_desc& s, const Tuning& tun
       const int32_t P = static_cast<int32_t>(s.h_context_lens[bl.b] - T);
       for (int32_t hk = 0; hk < g.kv_heads; ++hk)
         plan->prefill.push_back(PrefillItem{row_base[bl.b], T, P, bl.q0, PackHkSplit(hk, pc.split),
-                                            s.h_table_offsets[bl.b], pc.kb, pc.ke});
+                                            s.h_table_offsets[bl.b], pc.kb, pc.ke, bl.b});
     }
   }
   FinishPlan(g, tune, plan, true, &skip);

@@ -117,6 +117,14 @@ struct PrefillItem {
   int32_t table_off;
   int32_t key_begin;
   int32_t key_end;
+  int32_t seq;       // sequence of the step
+};
+
+// Where one sequence's contiguous [Hkv, L, d] K and V lie (calls over separate
+// per-sequence caches): device addresses and the bytes between kv heads.
+struct SeqBase {
+  uint64_t k, v;
+  int64_t head_bytes;
 };
 
 // Rows per joint item: at most 4, and at most 16 / g, so that the item's
@@ -162,6 +170,7 @@ struct Plan {
   std::vector<Q8Group> q8_groups;   // scaled-KV append groups (INT8/FP8 with slots)
   std::vector<int32_t> q8_rows;     // row indices of the groups, in offset order
   int32_t q8_max_rows = 0;          // rows of the largest append group
+  std::vector<SeqBase> seqs;        // per-sequence caches (empty: one pair of slabs)
   int64_t partials = 0;             // sum over rows of nsplit * Hkv
   int64_t max_length = 0;           // longest visible length (largest position + 1)
   int32_t split_tokens = 0;         // base split length chosen for this step
@@ -207,14 +216,14 @@ struct PrefillShape {
   int32_t slots = 512;
   int32_t min_tiles = 8;
   double split = 2.0;
+  int32_t min_rows = 16;  // rows of the shortest chunk it takes
 };
 
 // Validates the step (lengths, CSR offsets, every table id and slot in range)
-// and builds the plan. Chunks of at least kMinPrefillRows rows go to the
+// and builds the plan. Chunks of at least shape.min_rows rows go to the
 // matrix-core chunk kernel when one covers the geometry (shape.rows > 0;
 // Tuning::prefill = false keeps every row on the decode kernels); their rows
 // get nsplit = 0.
-constexpr int32_t kMinPrefillRows = 16;
 constexpr int32_t kPrefillTile = 32;       // keys per prefill tile
 // head_major: K/V are one contiguous [Hkv, L, d] cache read through an
 // identity table (block_stride = bs * d, kv heads L * d apart), so the slab
