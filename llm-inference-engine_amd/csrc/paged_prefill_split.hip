@@ -40,7 +40,9 @@
 // The planes of a non-finite V value cannot go through the matrix cores: the
 // zero probability of a masked key would turn it into NaN in rows that do not
 // attend it. A tile holding one takes a VALU pass that adds each row's
-// attended keys only.
+// attended keys only. Nor can those of a non-finite fp32 or bf16 K value,
+// whose products with q's planes can be infinities of both signs: a tile
+// holding one forms its scores by fp32 multiply-adds of the whole values.
 #include <climits>
 
 #include "decode_common.h"
@@ -159,7 +161,7 @@ void PrefillSplitMfma(PrefillParams p) {
 
   __shared__ __align__(16) unsigned char tiles[NBUF][2 * KP * PLANE];
   __shared__ __align__(16) float tile_scale[NBUF][4];  // K, V scales of the tile's halves
-  __shared__ __align__(16) int tile_odd[NBUF][WAVES];  // non-finite V seen by a wavefront
+  __shared__ __align__(16) int tile_odd[NBUF][WAVES];  // non-finite V (1), K (2) a wavefront saw
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -262,9 +264,9 @@ void PrefillSplitMfma(PrefillParams p) {
       }
     }
   };
-  // Convert a loaded tile into planes in LDS; notes non-finite V values.
+  // Convert a loaded tile into planes in LDS; notes non-finite values.
   auto store_tile = [&](const Stage& st, int buf) __attribute__((always_inline)) {
-    bool odd = false;
+    bool odd = false, oddk = false;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       const bool isv = is_v(i);
@@ -274,30 +276,29 @@ void PrefillSplitMfma(PrefillParams p) {
         uint32_t lo[KP], hi[KP];
         SplitPair(__uint_as_float(x[0]), __uint_as_float(x[1]), pf, lo);
         SplitPair(__uint_as_float(x[2]), __uint_as_float(x[3]), pf, hi);
-        if (isv) {
-          uint32_t top = 0;
+        uint32_t top = 0;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) top = max(top, x[e] & 0x7FFFFFFFu);
-          if (top >= kBf16Overflow) {
-            // Non-finite values whole in plane 0 (a NaN's payload quieted),
-            // finite ones cut towards zero, which cannot overflow.
-            odd = true;
-            uint32_t cut[4][KP];
+        for (int e = 0; e < 4; ++e) top = max(top, x[e] & 0x7FFFFFFFu);
+        if (top >= kBf16Overflow) {
+          // Non-finite values whole in plane 0 (a NaN's payload quieted),
+          // finite ones cut towards zero, which cannot overflow.
+          odd = odd | isv;
+          oddk = oddk | !isv;
+          uint32_t cut[4][KP];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const bool fin = (x[e] & 0x7FFFFFFFu) < 0x7F800000u;
-              float r = __uint_as_float(x[e]);
-#pragma unroll
-              for (int a = 0; a < KP; ++a) {
-                cut[e][a] = a == 0 && !fin ? Fp32ToBf16Bits(r) : __float_as_uint(r) >> 16;
-                r = fin ? r - __uint_as_float(cut[e][a] << 16) : 0.f;
-              }
-            }
+          for (int e = 0; e < 4; ++e) {
+            const bool fin = (x[e] & 0x7FFFFFFFu) < 0x7F800000u;
+            float r = __uint_as_float(x[e]);
 #pragma unroll
             for (int a = 0; a < KP; ++a) {
-              lo[a] = cut[0][a] | cut[1][a] << 16;
-              hi[a] = cut[2][a] | cut[3][a] << 16;
+              cut[e][a] = a == 0 && !fin ? Fp32ToBf16Bits(r) : __float_as_uint(r) >> 16;
+              r = fin ? r - __uint_as_float(cut[e][a] << 16) : 0.f;
             }
+          }
+#pragma unroll
+          for (int a = 0; a < KP; ++a) {
+            lo[a] = cut[0][a] | cut[1][a] << 16;
+            hi[a] = cut[2][a] | cut[3][a] << 16;
           }
         }
 #pragma unroll
@@ -305,11 +306,12 @@ void PrefillSplitMfma(PrefillParams p) {
           *reinterpret_cast<uint2*>(dst + a * PLANE + vc * 8) = make_uint2(lo[a], hi[a]);
       } else if constexpr (KV == EHIP_KV_BF16) {
         *reinterpret_cast<uint4*>(dst + vc * 16) = make_uint4(x[0], x[1], x[2], x[3]);
-        if (isv) {
+        bool over = false;
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            odd = odd | ((((x[e] & 0x7FFF7FFFu) + 0x00800080u) & 0x80008000u) != 0);
-        }
+        for (int e = 0; e < 4; ++e)
+          over = over | ((((x[e] & 0x7FFF7FFFu) + 0x00800080u) & 0x80008000u) != 0);
+        odd = odd | (over & isv);
+        oddk = oddk | (over & !isv);
       } else {
         uint32_t w[8];
 #pragma unroll
@@ -348,7 +350,7 @@ void PrefillSplitMfma(PrefillParams p) {
         }
       }
     }
-    const int any = __any(odd);
+    const int any = (__any(odd) ? 1 : 0) | (__any(oddk) ? 2 : 0);
     if (lane == 0) tile_odd[buf][wave] = any;
   };
 
@@ -452,7 +454,41 @@ void PrefillSplitMfma(PrefillParams p) {
       const int4 x = *reinterpret_cast<const int4*>(&tile_odd[buf][i]);
       oddw |= x.x | x.y | x.z | x.w;
     }
-    const bool odd = __builtin_amdgcn_readfirstlane(oddw) != 0;
+    const int oddf = __builtin_amdgcn_readfirstlane(oddw);
+    const bool odd = (oddf & 1) != 0;
+    if constexpr (!kScaled) {
+      if (oddf & 2) {
+        // Non-finite K in the tile: each key's products over this lane's
+        // elements of q (read again: the loop keeps few registers), added over
+        // the vector's four lanes.
+#pragma unroll 1
+        for (int tok = 0; tok < kTile; ++tok) {
+          float sum[HB];
+#pragma unroll
+          for (int hh = 0; hh < HB; ++hh) sum[hh] = 0.f;
+#pragma unroll 1
+          for (int e = 8 * kq; e < D; e += e % 8 == 7 ? 25 : 1) {
+            float kv = 0.f;
+#pragma unroll
+            for (int a = KP - 1; a >= 0; --a)
+              kv += static_cast<float>(
+                  *reinterpret_cast<const __bf16*>(kb + a * PLANE + tok * PITCH + 2 * e));
+#pragma unroll
+            for (int hh = 0; hh < HB; ++hh)
+              sum[hh] = fmaf(p.q[(int64_t{it.row_base + q0 + vrow[hh]} * p.heads + hk * g +
+                                  vhead[hh]) * D + e],
+                             kv, sum[hh]);
+          }
+#pragma unroll
+          for (int hh = 0; hh < HB; ++hh) {
+            const float x = RowReduce(sum[hh], [](float a, float b) { return a + b; });
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+              if (tok == 16 * (j >> 2) + 4 * kq + (j & 3)) s[hh][j >> 2][j & 3] = x;
+          }
+        }
+      }
+    }
 
     // The operand of lane (n, kq) is V[token][16 nb + n] over the tokens its
     // probabilities cover: two transposed reads per plane. A group of column

@@ -127,3 +127,16 @@ def test_rows_before_a_non_finite_value_stay_clean(gctx, ehip_mod, orc, bf16, d,
     assert not np.isfinite(got[hit]).any()
     if not np.isnan(bad):
         assert (got[hit] == (np.inf if bad > 0 else -np.inf)).all()
+
+
+@pytest.mark.parametrize("bf16,d", [(False, 64), (False, 128), (True, 64)])
+def test_keys_at_minus_infinity_take_no_part(gctx, ehip_mod, orc, bf16, d):
+    """A K element of -inf against positive queries scores -inf: its key has
+    probability 0, as one scored -1e30 in the reference."""
+    c = make_case(orc, bf16, 14, 2, d, 16, [(70, 40)], seed=5 + d)
+    pos, col = 83, 9
+    c.q[:, :, col] = np.abs(c.q[:, :, col]) + 0.1
+    c.k[c.tables[0][pos // 16], 1, pos % 16, col] = -np.inf
+    c.ks[0][1, pos, col] = -1e30
+    got = run(gctx, ehip_mod, orc, c)
+    assert rel_norm(got, reference(orc, c)) <= BAR
