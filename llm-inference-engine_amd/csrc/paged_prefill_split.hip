@@ -740,6 +740,14 @@ PrefillShape PrefillSplitShape(int kv_dtype, int d, int group, int64_t block_str
   s.slots = 256 * 8 / SplitWaves(kv_dtype);  // two wavefronts per SIMD
   s.min_tiles = 4;
   s.split = 1.0;
+  // Beside decode rows the chunks cost a launch of their own (~7 us a layer),
+  // which little work does not earn back. Four layers with 2 or 12 decode rows
+  // and 1 or 3 chunks of 16-204 rows, this kernel's time over the decode
+  // kernels', by pairs x heads x d: g = 4, fp32 1.05-1.38 at 21-24M and 0.58-0.71
+  // at 39-56M, FP8 1.05-1.21 and 0.82-0.95; g = 7, fp32 1.10 at 68M, 1.06 at 94M
+  // and 0.78-0.96 at 132-162M; g = 8, INT8 1.08-1.23 at 42-48M, 0.84-0.91 at
+  // 154-170M. Steps without decode rows: 0.2-1.0, whatever the work.
+  s.min_work = group > 4 ? int64_t{1} << 27 : int64_t{1} << 25;
   return s;
 }
 

@@ -81,6 +81,7 @@ Tuning ReadTuning() {
   if (const char* v = std::getenv("EHIP_SPLIT_EVEN")) t.split_even = v[0] == '1' ? 1 : v[0] == '0' ? 0 : -1;
   t.joint = flag("EHIP_NO_JOINT", '1');
   t.prefill = flag("EHIP_PREFILL", '0');
+  if (const char* v = std::getenv("EHIP_PREFILL")) t.prefill_all = std::strcmp(v, "1") == 0;
   if (const char* v = std::getenv("EHIP_PREFILL_SPLIT")) t.prefill_split = std::strtod(v, nullptr);
   if (const char* v = std::getenv("EHIP_PREFILL_TILES")) {
     const long x = std::strtol(v, nullptr, 10);
@@ -618,7 +619,20 @@ int BuildPlan(const ehip_geometry& g, const ehip_step_desc& s, const Tuning& tun
 
   // Chunks big enough for the MFMA prefill kernel leave the decode partition.
   std::vector<int32_t> skip(plan->rows.size(), 0);
-  if (prefill_rows > 0 && tune.prefill) {
+  bool chunk_kernel = prefill_rows > 0 && tune.prefill;
+  if (chunk_kernel && shape.min_work > 0 && !tune.prefill_all) {
+    int64_t pairs = 0;  // below 2^24 rows x 2^31 keys
+    bool decodes = false;
+    for (int32_t b = 0; b < B; ++b) {
+      const int64_t T = s.h_query_lens[b];
+      if (T < shape.min_rows)
+        decodes = true;
+      else
+        pairs += T * (s.h_context_lens[b] - T) + T * (T + 1) / 2;
+    }
+    chunk_kernel = !decodes || pairs >= shape.min_work / (int64_t{g.heads} * g.head_dim);
+  }
+  if (chunk_kernel) {
     struct Block { int32_t b, q0, keys; };
     std::vector<Block> blocks;
     std::vector<int32_t> row_base(B + 1, 0);

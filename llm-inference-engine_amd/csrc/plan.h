@@ -43,6 +43,7 @@ struct Tuning {
                                // always / never (default: when items <= the item target)
   bool joint = true;           // EHIP_NO_JOINT=1: no joint items over shared prefixes
   bool prefill = true;         // EHIP_PREFILL=0: chunk rows stay on the decode kernels
+  bool prefill_all = false;    // EHIP_PREFILL=1: small chunks beside decode rows leave them too
   double prefill_split = -1;   // EHIP_PREFILL_SPLIT: key-split threshold in shares (0: none;
                                // default: the chunk kernel's own, PrefillShape)
   int32_t prefill_tiles = 0;   // EHIP_PREFILL_TILES: least tiles of a key split (0: the kernel's)
@@ -209,14 +210,17 @@ int32_t SingleRowSplitTokens(const ehip_geometry& g, int64_t length, const Tunin
 
 // How the step's chunk kernel takes its work: query rows per item (0: no
 // kernel, chunk rows stay on the decode kernels), workgroups resident at once,
-// the least tiles of a key split, and the shares of the step's tiles past
-// which a block is split.
+// the least tiles of a key split, the shares of the step's tiles past which a
+// block is split, the shortest chunk, and the work (attended pairs x heads x d
+// of the step's chunks) below which a step with decode rows keeps its chunks on
+// their launch.
 struct PrefillShape {
   int rows = 0;
   int32_t slots = 512;
   int32_t min_tiles = 8;
   double split = 2.0;
-  int32_t min_rows = 16;  // rows of the shortest chunk it takes
+  int32_t min_rows = 16;
+  int64_t min_work = 0;
 };
 
 // Validates the step (lengths, CSR offsets, every table id and slot in range)

@@ -2,7 +2,8 @@
 fp32 K/V and the bf16 shapes the bf16 block kernel does not cover, at the
 edges of its tiles (16-vector blocks, 32-key tiles, key splits), against the
 oracle's restatement of PrefillAttentionVarlenF32 and against the same step
-with every row on the decode kernels (EHIP_PREFILL=0).
+with every row on the decode kernels (EHIP_PREFILL=0; =1 keeps small chunks
+beside a decode row on the chunk kernel).
 
 Bars: 1e-4 relative per output vector, the decode kernels' fp32 bar: the
 products left out of the plane splits are below 3 * 2^-24 of |q||k| (and
@@ -91,7 +92,7 @@ def reference(orc, c):
 def test_chunks_match_the_oracle(ehip_mod, orc, tctx, bf16, H, Hkv, d, bs, chunks):
     c = make_case(orc, bf16, H, Hkv, d, bs, chunks, seed=H + d + bs + chunks[0][0])
     ref = reference(orc, c)
-    ctx = tctx()
+    ctx = tctx(EHIP_PREFILL="1")
     got = run(ctx, ehip_mod, orc, c)
     assert rel_norm(got, ref) <= BAR, rel_norm(got, ref)
     if chunks[0][1] == 700:  # 24 tiles: cut into key splits
@@ -101,26 +102,28 @@ def test_chunks_match_the_oracle(ehip_mod, orc, tctx, bf16, H, Hkv, d, bs, chunk
 
 
 @pytest.mark.parametrize("bf16,d", [(False, 64), (False, 128), (True, 64)])
-def test_chunk_operands_at_any_alignment(gctx, ehip_mod, orc, bf16, d):
+def test_chunk_operands_at_any_alignment(tctx, ehip_mod, orc, bf16, d):
     """q, slabs and outputs 4 bytes off a 16-byte boundary, as the decode
     kernels take them (the decode row after the chunk takes another of them
     there)."""
+    ctx = tctx(EHIP_PREFILL="1")
     c = make_case(orc, bf16, 14, 2, d, 16, [(45, 20)], seed=d)
-    off, on = run(gctx, ehip_mod, orc, c, shift=4), run(gctx, ehip_mod, orc, c)
+    off, on = run(ctx, ehip_mod, orc, c, shift=4), run(ctx, ehip_mod, orc, c)
     assert np.array_equal(off[:45], on[:45])
     assert rel_norm(off, on) <= BAR
 
 
 @pytest.mark.parametrize("bf16,d", [(False, 64), (False, 128), (True, 64)])
 @pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
-def test_rows_before_a_non_finite_value_stay_clean(gctx, ehip_mod, orc, bf16, d, bad):
+def test_rows_before_a_non_finite_value_stay_clean(tctx, ehip_mod, orc, bf16, d, bad):
     """A non-finite V element reaches the rows that attend its key, in its
     column, and no other output."""
+    ctx = tctx(EHIP_PREFILL="1")
     c = make_case(orc, bf16, 14, 2, d, 16, [(70, 40)], seed=3 + d)
-    clean = run(gctx, ehip_mod, orc, c)
+    clean = run(ctx, ehip_mod, orc, c)
     pos, col = 83, 9  # key 83 of the chunk's sequence: rows 43.. attend it
     c.v[c.tables[0][pos // 16], 1, pos % 16, col] = bad
-    got = run(gctx, ehip_mod, orc, c)
+    got = run(ctx, ehip_mod, orc, c)
     hit = np.zeros(got.shape, bool)
     hit[43:70, 7:, col] = True
     assert rel_norm(got[~hit][None], clean[~hit][None]) <= BAR
@@ -130,13 +133,14 @@ def test_rows_before_a_non_finite_value_stay_clean(gctx, ehip_mod, orc, bf16, d,
 
 
 @pytest.mark.parametrize("bf16,d", [(False, 64), (False, 128), (True, 64)])
-def test_keys_at_minus_infinity_take_no_part(gctx, ehip_mod, orc, bf16, d):
+def test_keys_at_minus_infinity_take_no_part(tctx, ehip_mod, orc, bf16, d):
     """A K element of -inf against positive queries scores -inf: its key has
     probability 0, as one scored -1e30 in the reference."""
+    ctx = tctx(EHIP_PREFILL="1")
     c = make_case(orc, bf16, 14, 2, d, 16, [(70, 40)], seed=5 + d)
     pos, col = 83, 9
     c.q[:, :, col] = np.abs(c.q[:, :, col]) + 0.1
     c.k[c.tables[0][pos // 16], 1, pos % 16, col] = -np.inf
     c.ks[0][1, pos, col] = -1e30
-    got = run(gctx, ehip_mod, orc, c)
+    got = run(ctx, ehip_mod, orc, c)
     assert rel_norm(got, reference(orc, c)) <= BAR

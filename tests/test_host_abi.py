@@ -606,3 +606,16 @@ def test_plan_every_row_keeps_a_range_ending_at_its_last_key(ehip_mod, L):
         assert (own[:, 5] == L).sum() == 8, f"row {r}: no range of its own ending at {L}"
     joint = items[items[:, 1] >= 0]
     assert joint[:, 5].max() <= (L - 1) // bs * bs
+
+
+@pytest.mark.parametrize("H,T,past", [(32, 16, 0), (32, 90, 0), (64, 170, 0), (64, 181, 0)])
+def test_small_chunks_beside_decode_rows_stay_with_them(ehip_mod, H, T, past):
+    """fp32 chunks leave a step's decode kernels from 2^25 attended pairs x
+    heads x d on (g = 4; 2^27 at g = 8), alone at any work."""
+    E = ehip_mod
+    g = geom(E, heads=H, kv_heads=8, head_dim=128, kv_dtype=E.KV_F32, slab_blocks=64)
+    both = simple_step(E, [T + past, 40], qlens=np.array([T, 1], np.int32))
+    alone = simple_step(E, [T + past], qlens=np.array([T], np.int32))
+    work = T * (T + 1) // 2 * H * 128
+    assert (len(prefill_items(E, g, both)) > 0) == (work >= 1 << (27 if H == 64 else 25))
+    assert len(prefill_items(E, g, alone)) > 0
