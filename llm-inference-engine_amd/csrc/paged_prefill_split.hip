@@ -70,6 +70,10 @@ __device__ __forceinline__ Vec16 LoadGlobal(uint64_t at) {
 
 constexpr int kTile = 32;  // keys per tile
 constexpr float kRefSlack = 8.f;
+// Softmax references below this size take the exponents as one fused
+// multiply-add; a larger one rounds further from its score than an exponent's
+// unit, so there the score is rounded first, as the reference was.
+constexpr float kFusedRef = 16777216.f;
 constexpr int kPP = 3;  // planes of the probabilities
 
 template <int KV>
@@ -107,6 +111,12 @@ __device__ __forceinline__ float RowReduce(float x, Op op) {
   const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false,
                                                   false);
   return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+// a * b rounded by itself (not fused into a sum it enters).
+__device__ __forceinline__ float Product(float a, float b) {
+#pragma clang fp contract(off)
+  return a * b;
 }
 
 // The pair (x, y) as N bf16 planes, one packed word each: a packed RNE
@@ -510,7 +520,7 @@ void PrefillSplitMfma(PrefillParams p) {
     // t[hh][j]: exponent of key k0 + 16 (j / 4) + 4 kq + j % 4, relative to the
     // row's reference; masked keys are -inf. The reference moves only past a
     // slack of 2^8 (lazy rescaling), so most tiles need no row reduction.
-    float t[HB][8], tmax[HB];
+    float t[HB][8];
     bool need = false;
 #pragma unroll
     for (int hh = 0; hh < HB; ++hh) {
@@ -525,23 +535,32 @@ void PrefillSplitMfma(PrefillParams p) {
       float tm = -INFINITY;
 #pragma unroll
       for (int j = 0; j < 8; ++j) tm = fmaxf(tm, t[hh][j]);
-      tmax[hh] = tm;
-      need = need || ref[hh] == -INFINITY || tm > kRefSlack;
+      need = need || !(fabsf(ref[hh]) < kFusedRef) || tm > kRefSlack;
     }
     if (__any(need)) {
+      // The reference moves to the row's largest score, and the exponents are
+      // formed from the scores again: the first ones would keep the rounding
+      // at the jump's size.
       bool moved = false;
       float alpha[HB];
 #pragma unroll
       for (int hh = 0; hh < HB; ++hh) {
-        const float tr = RowReduce(tmax[hh], [](float a, float b) { return fmaxf(a, b); });
-        const bool unset = ref[hh] == -INFINITY;
-        const bool mv = tr != -INFINITY && (unset || tr > kRefSlack);
-        const float d = mv ? tr : 0.f;
-        alpha[hh] = unset ? 1.f : Exp2(-d);
-        ref[hh] = mv ? (unset ? 0.f : ref[hh]) + tr : ref[hh];
-        moved = moved || mv;
+        float x[8], top = -INFINITY;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) t[hh][j] -= d;
+        for (int j = 0; j < 8; ++j) {
+          x[j] = Product(s[hh][j >> 2][j & 3], ks[j >> 2]);
+          top = fmaxf(top, t[hh][j] == -INFINITY ? -INFINITY : x[j]);
+        }
+        top = RowReduce(top, [](float a, float b) { return fmaxf(a, b); });
+        const bool mv = top > ref[hh] + kRefSlack;
+        alpha[hh] = mv && ref[hh] != -INFINITY ? Exp2(ref[hh] - top) : 1.f;
+        ref[hh] = mv ? top : ref[hh];
+        moved = moved || mv;
+        const bool fused = fabsf(ref[hh]) < kFusedRef;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          if (t[hh][j] != -INFINITY)
+            t[hh][j] = fused ? fmaf(s[hh][j >> 2][j & 3], ks[j >> 2], -ref[hh]) : x[j] - ref[hh];
         l[hh] *= alpha[hh];
       }
       if (__any(moved)) {

@@ -78,6 +78,23 @@ def run(ctx, ehip_mod, orc, c, shift=0):
     return raw[shift:].view(np.float32).reshape(c.q.shape)
 
 
+def exact(q, ks, vs, qlens, lens, scale):
+    """The chunks' attention in 64 bits: q [rows, H, d], per sequence K and V
+    [Hkv, L, d]. Rows of a sequence sit at its last positions."""
+    q = np.asarray(q, np.float64)
+    H = q.shape[1]
+    out, at = np.empty_like(q), 0
+    for k, v, t, n in zip(ks, vs, qlens, lens):
+        k = np.repeat(np.asarray(k, np.float64), H // k.shape[0], axis=0)
+        v = np.repeat(np.asarray(v, np.float64), H // v.shape[0], axis=0)
+        s = q[at:at + t].transpose(1, 0, 2) @ k.transpose(0, 2, 1) * scale
+        s[:, np.arange(n)[None, :] > np.arange(n - t, n)[:, None]] = -np.inf
+        p = np.exp(s - s.max(axis=2, keepdims=True))
+        out[at:at + t] = ((p @ v) / p.sum(axis=2, keepdims=True)).transpose(1, 0, 2)
+        at += t
+    return out
+
+
 def reference(orc, c):
     cu = np.concatenate([[0], np.cumsum(c.qlens)]).astype(np.int32)
     return orc.prefill_varlen(c.q, cu, c.ks, c.vs, c.H, c.Hkv, c.d, scale_for(c.d), isa=1)
@@ -144,3 +161,94 @@ def test_keys_at_minus_infinity_take_no_part(tctx, ehip_mod, orc, bf16, d):
     c.ks[0][1, pos, col] = -1e30
     got = run(ctx, ehip_mod, orc, c)
     assert rel_norm(got, reference(orc, c)) <= BAR
+
+
+def scaled_codes(rng, fp8, shape):
+    """Random INT8 codes, or E4M3 ones of finite values, as bytes; and the
+    values they stand for."""
+    if not fp8:
+        codes = rng.integers(-127, 128, shape).astype(np.int8)
+        return codes.view(np.uint8), codes.astype(np.float64)
+    codes = rng.integers(0, 256, shape).astype(np.uint8)
+    codes[(codes & 0x7F) == 0x7F] = 0
+    return codes, e4m3(codes)
+
+
+def e4m3(codes):
+    c = codes.astype(np.int32)
+    e, m = c >> 3 & 15, c & 7
+    mag = np.where(e == 0, np.ldexp(m / 8.0, -6), np.ldexp(1 + m / 8.0, e - 7))
+    mag = np.where((c & 0x7F) == 0x7F, np.nan, mag)
+    return np.where(c & 0x80, -mag, mag)
+
+
+def run_scaled(ctx, ehip_mod, fp8, H, Hkv, d, bs, T, P, seed, edit=None):
+    """One chunk of T rows after P keys over INT8 or FP8 K/V with random codes
+    and scales; edit(q, k, v, ks, vs) changes q, codes and scales first, the
+    sequence's block j being block j of the slab. Returns the kernel's rows and
+    q and the dequantised K and V [Hkv, L, d]."""
+    rng = np.random.default_rng(seed)
+    L = T + P
+    nb = -(-L // bs)
+    q = rng.standard_normal((T, H, d)).astype(np.float32)
+    k, v = (scaled_codes(rng, fp8, (nb, Hkv, bs, d))[0] for _ in "kv")
+    top = 448.0 if fp8 else 127.0
+    ks, vs = ((rng.uniform(1.5, 3.5, (nb, Hkv)) / top).astype(np.float32) for _ in "kv")
+    if edit:
+        edit(q, k, v, ks, vs)
+
+    def values(codes, sc):
+        x = e4m3(codes) if fp8 else codes.view(np.int8).astype(np.float64)
+        with np.errstate(invalid="ignore"):
+            x = x * sc.astype(np.float64)[:, :, None, None]
+        return x.transpose(1, 0, 2, 3).reshape(Hkv, nb * bs, d)[:, :L]
+
+    bufs = [ctx.to_device(x) for x in (q, k, v, ks, vs)] + [ctx.alloc(q.nbytes)]
+    fmt = "fp8" if fp8 else "int8"
+    dt = ehip_mod.KV_FP8 if fp8 else ehip_mod.KV_INT8
+    g = ehip_mod.geometry(H, Hkv, d, bs, dt, nb, scale_for(d))
+    st = ehip_mod.StepArrays([T], [L], [np.arange(nb, dtype=np.int32)])
+    assert ctx.step_upload(g, st) == 0, ctx.last_error()
+    assert getattr(ctx, "step_attention_" + fmt)(*bufs) == 0, ctx.last_error()
+    ctx.sync()
+    got = bufs[-1].download(np.float32, q.shape)
+    for b in bufs:
+        b.free()
+    return got, q, values(k, ks), values(v, vs)
+
+
+@pytest.mark.parametrize("M", [1e3, 1e5, 1e30])
+@pytest.mark.parametrize("T,P", [(33, 64), (40, 700)], ids=["whole", "splits"])
+@pytest.mark.parametrize("kv,d", [("f32", 64), ("f32", 128), ("bf16", 64), ("int8", 128),
+                                  ("int8", 64), ("fp8", 128), ("fp8", 64)])
+def test_scores_that_jump_between_tiles(tctx, ehip_mod, orc, kv, d, T, P, M):
+    """A row's first 64 keys score about -M, its others as usual: the softmax
+    reference jumps by M at its third tile, and the scores there keep their
+    differences. Bars against 64 bits: 2e-6 (planes of 24 bits: about 2^-21 in
+    a score of a few units, as far in a probability); over FP8 q has two planes,
+    2^-18 of |q||k| is left out, 2e-5."""
+    ctx = tctx(EHIP_PREFILL="1")
+    low = -M / scale_for(d)
+    if kv in ("f32", "bf16"):
+        c = make_case(orc, kv == "bf16", 14, 2, d, 16, [(T, P)], seed=d + T)
+        c.q[:T, :, 0] = 1.0
+        c.ks[0][:, :, 0] = 0.0
+        c.ks[0][:, :64, 0] = low
+        if kv == "bf16":
+            c.ks[0] = orc.bf16_bits_to_f32(orc.to_bf16_bits(c.ks[0]))
+        for s in range(T + P):
+            c.k[c.tables[0][s // 16], :, s % 16] = c.ks[0][:, s]
+        got = run(ctx, ehip_mod, orc, c)[:T]
+        ref = exact(c.q[:T], c.ks[:1], c.vs[:1], [T], [T + P], scale_for(d))
+    else:
+        def edit(q, k, v, ks, vs):
+            q[:, :, 0] = 1.0
+            k[:, :, :, 0] = 0
+            k[:4] = 0
+            k[:4, :, :, 0] = 0xFE if kv == "fp8" else 0x81  # -448, -127
+            ks[:4] = -low / (448.0 if kv == "fp8" else 127.0)
+
+        got, q, k, v = run_scaled(ctx, ehip_mod, kv == "fp8", 8, 2, d, 16, T, P, d + T, edit)
+        ref = exact(q, [k], [v], [T], [T + P], scale_for(d))
+    bar = 2e-5 if kv == "fp8" else 2e-6
+    assert rel_norm(got, ref) <= bar, rel_norm(got, ref)
