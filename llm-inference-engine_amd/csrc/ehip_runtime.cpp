@@ -817,7 +817,7 @@ namespace {
 // vectors empty, but a plan, upload and launch of its own cost ~20 us: six
 // members of 1-400 rows over up to 1000 keys 118 -> 45 us a call). *done stays
 // false where the kernel does not cover the shape or the call exceeds one
-// plan's limits, and for one short member, which the decode kernels serve.
+// plan's limits, and for one member, which has one plan and launch either way.
 int VarlenOneLaunch(ehip_ctx* ctx, const float* d_q, const int32_t* cu, int64_t num_seqs,
                     const float* const* k_seqs, const float* const* v_seqs,
                     const int64_t* l_dims, float* d_out, int64_t heads, int64_t kv_heads,
@@ -825,10 +825,10 @@ int VarlenOneLaunch(ehip_ctx* ctx, const float* d_q, const int32_t* cu, int64_t 
   constexpr int32_t kRun = 16;
   ehip::PrefillShape shape = ehip::PrefillSplitShape(
       EHIP_KV_F32, static_cast<int>(d), static_cast<int>(heads / kv_heads), kRun * d);
-  if (shape.rows == 0 || !ctx->tune.prefill || cu[num_seqs] > (1 << 24) ||
-      (num_seqs == 1 && cu[1] < shape.min_rows))
+  if (shape.rows == 0 || !ctx->tune.prefill || cu[num_seqs] > (1 << 24) || num_seqs == 1)
     return EHIP_OK;
   shape.min_rows = 1;
+  shape.min_work = 0;  // every member on this kernel, whatever its work
   int64_t blocks = 0, longest = 0;
   for (int64_t b = 0; b < num_seqs; ++b) {
     const int64_t n = (l_dims[b] + kRun - 1) / kRun;

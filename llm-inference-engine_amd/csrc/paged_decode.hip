@@ -31,11 +31,9 @@ namespace ehip {
 namespace {
 
 constexpr int kWavesPerBlock = 4;
-// Steps with at most this many (row, kv head) units take the workgroup-per-unit
-// kernel (4 or 8 wavefronts each, 2048 wavefronts at most).
-constexpr int64_t kWgMaxUnits = 256;
-// ... and only when no row needs more than this many 32-key tiles per
-// wavefront: past that, the split-KV path (more wavefronts on a long row,
+// Steps with at most kWgMaxUnits (row, kv head) units take the
+// workgroup-per-unit kernel, and only when no row needs more than this many
+// 32-key tiles per wavefront: past that, the split-KV path (more wavefronts on a long row,
 // merged by a second kernel) measured faster (C2: rows up to 2049 keys,
 // 32.6 against 39.0 us per layer; C1: one 513-key row, 17.3 against 22.0 us).
 constexpr int kWgMaxTilesPerWave = 6;

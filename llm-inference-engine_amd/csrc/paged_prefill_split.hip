@@ -751,6 +751,50 @@ constexpr int SplitBlocks(int kv_dtype, int d) { return kv_dtype != EHIP_KV_F32 
 
 }  // namespace
 
+namespace {
+
+// Steps of few rows that the decode kernels take in one launch and finish
+// before this kernel, whose chunks past four tiles need the split merge too.
+// us a layer, decode kernels / this kernel, by the step's longest context:
+//   fp32, d = 64: g = 1 (24 rows, 8 kv heads) 7.4/8.3 at 24 keys, 12.7/14.9 at
+//     760, 13.4/14.6 at 800, 15.4/15.0 at 1100; g = 4 (32 rows) 8.3/9.6 at 32, 16.8/18.0 at 760,
+//     19.4/17.5 at 900; g = 7 (32 rows, 2 kv heads) 11.2/10.3 at 64, 12.0/13.4
+//     at 128, 12.4/16.3 at 200, 16.4/17.3 at 500, 19.1/17.6 at 600; g = 8 (32
+//     rows, 2) 10.8/10.3 at 64, 11.1/12.5 at 80, 14.5/16.7 at 200, 17.2/17.0 at
+//     300.
+//   fp32, d = 128: g = 2 (24 rows, 8) 8.1/10.7 at 24, 19.1/19.6 at 700, 22.5/19.2
+//     at 900; g = 7 (32 rows, 2) 17.0/14.5 at 64, 15.5/18.3 at 80, 17.4/22.5 at
+//     200, 24.2/22.9 at 300; g = 8 (24 rows, 8) 12.2/13.1 at 24, 18.9/22.3 at
+//     200, 23.8/24.6 at 300, 28.4/25.1 at 400. (g = 4 has no workgroup per row
+//     there: 15.3/13.8 at 48, 68/24 at 200.)
+//   FP8, 8 kv heads: d = 64, g = 4 8.5/9.5 at 24, 9.3/10.2 at 64, 10.4/11.6 at 96
+//     (32 rows); g = 8 9.0/9.9 at 16, 10.4/10.5 at 48; d = 128, g = 4 8.4/9.2 at
+//     16, 10.1/9.5 at 36. INT8, d = 64, g = 4: 9.0/9.7 at 32, 11.1/11.7 at 80;
+//     d = 128: 9.7/9.5 at 24. Past about 350 units or below 128 (2 kv heads) the
+//     two are within 5%, this kernel ahead.
+void SetFewRows(int kv_dtype, int d, int group, PrefillShape* s) {
+  const bool d64 = d == 64, fp8 = kv_dtype == EHIP_KV_FP8;
+  if (kv_dtype == EHIP_KV_F32) {
+    s->few_lo = 1;
+    s->few_hi = kWgMaxUnits;
+    if (group == 1 || group == 2 || (group == 4 && d64))
+      s->few_keys_hi = group == 1 && d64 ? 896 : 768;
+    else if (group == 7)
+      s->few_keys_lo = 64, s->few_keys_hi = d64 ? 512 : 256;
+    else if (group == 8)
+      s->few_keys_lo = d64 ? 64 : 0, s->few_keys_hi = d64 ? 256 : 384;
+  } else if (kv_dtype != EHIP_KV_BF16) {
+    s->few_lo = 128;
+    s->few_hi = 352;
+    if (group <= 4)
+      s->few_keys_hi = d64 ? 128 : fp8 ? 32 : 0;
+    else
+      s->few_keys_hi = d64 && fp8 ? 32 : 0;
+  }
+}
+
+}  // namespace
+
 PrefillShape PrefillSplitShape(int kv_dtype, int d, int group, int64_t block_stride) {
   PrefillShape s;
   if ((d != 64 && d != 128) || group < 1 || group > 64) return s;
@@ -767,6 +811,7 @@ PrefillShape PrefillSplitShape(int kv_dtype, int d, int group, int64_t block_str
   // and 0.78-0.96 at 132-162M; g = 8, INT8 1.08-1.23 at 42-48M, 0.84-0.91 at
   // 154-170M. Steps without decode rows: 0.2-1.0, whatever the work.
   s.min_work = group > 4 ? int64_t{1} << 27 : int64_t{1} << 25;
+  SetFewRows(kv_dtype, d, group, &s);
   return s;
 }
 

@@ -31,6 +31,11 @@ constexpr int32_t kMinSplit = 128;
 // attention call; C2, 500 items of 128 keys, is faster as it is).
 constexpr int64_t kSmallStepUnits = int64_t{128} * kMinSplit;
 constexpr int32_t kMaxSplitsPerRow = 64;  // bounds the merge a single wave performs
+// Keys by which a step's decode rows lengthen the contexts up to which few
+// rows stay on the decode kernels: their own launch beside a chunk kernel's
+// costs about 6 us a layer. 32 heads, 8 kv heads, d = 64, fp32, a 27-row chunk
+// at 830 keys and one decode row: 18.8 us a layer, 24.7 on both kernels.
+constexpr int32_t kDecodesFewKeys = 256;
 // Large steps (one item per resident wavefront would already mean ranges of
 // at least kLargeStep keys) take ranges of kLargeMin..kLargeMax keys. Measured
 // on MI355X (attention call per layer, one process, interleaved calls):
@@ -621,16 +626,29 @@ int BuildPlan(const ehip_geometry& g, const ehip_step_desc& s, const Tuning& tun
   std::vector<int32_t> skip(plan->rows.size(), 0);
   bool chunk_kernel = prefill_rows > 0 && tune.prefill;
   if (chunk_kernel && shape.min_work > 0 && !tune.prefill_all) {
-    int64_t pairs = 0;  // below 2^24 rows x 2^31 keys
+    int64_t pairs = 0, units = 0;  // pairs below 2^24 rows x 2^31 keys
     bool decodes = false;
     for (int32_t b = 0; b < B; ++b) {
       const int64_t T = s.h_query_lens[b];
+      const int64_t reads = T * (s.h_context_lens[b] - T) + T * (T + 1) / 2;
+      units += reads * g.kv_heads;
       if (T < shape.min_rows)
         decodes = true;
       else
-        pairs += T * (s.h_context_lens[b] - T) + T * (T + 1) / 2;
+        pairs += reads;
     }
-    chunk_kernel = !decodes || pairs >= shape.min_work / (int64_t{g.heads} * g.head_dim);
+    // Few rows, where the decode kernels write the outputs in one launch: fp32
+    // on a workgroup per unit, INT8 and FP8 with one range a row.
+    const int64_t few = total_rows * g.kv_heads;
+    const bool one_launch =
+        ScaledKv(g.kv_dtype)
+            ? plan->max_length <= (units < kSmallStepUnits ? kTile : kMinSplit)
+            : tune.decode_wg;
+    if (one_launch && few >= shape.few_lo && few <= shape.few_hi &&
+        plan->max_length > shape.few_keys_lo &&
+        plan->max_length <= shape.few_keys_hi + (decodes ? kDecodesFewKeys : 0))
+      chunk_kernel = false;
+    if (decodes && pairs < shape.min_work / (int64_t{g.heads} * g.head_dim)) chunk_kernel = false;
   }
   if (chunk_kernel) {
     struct Block { int32_t b, q0, keys; };

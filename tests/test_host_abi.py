@@ -619,3 +619,40 @@ def test_small_chunks_beside_decode_rows_stay_with_them(ehip_mod, H, T, past):
     work = T * (T + 1) // 2 * H * 128
     assert (len(prefill_items(E, g, both)) > 0) == (work >= 1 << (27 if H == 64 else 25))
     assert len(prefill_items(E, g, alone)) > 0
+
+
+@pytest.mark.parametrize("kv,H,Hkv,d,T,L,kept", [
+    ("KV_F32", 14, 2, 64, 16, 64, False), ("KV_F32", 14, 2, 64, 16, 65, True),
+    ("KV_F32", 14, 2, 64, 128, 512, True), ("KV_F32", 14, 2, 64, 16, 513, False),
+    ("KV_F32", 14, 2, 64, 129, 300, False), ("KV_F32", 32, 8, 64, 32, 768, True),
+    ("KV_F32", 32, 8, 64, 32, 769, False), ("KV_F32", 64, 8, 128, 16, 384, True),
+    ("KV_F32", 64, 8, 128, 16, 385, False), ("KV_F32", 32, 8, 128, 16, 100, False),
+    ("KV_F32", 24, 8, 64, 16, 100, False), ("KV_BF16", 14, 2, 64, 16, 200, False),
+    ("KV_FP8", 32, 8, 64, 16, 64, True), ("KV_FP8", 32, 8, 64, 16, 65, False),
+    ("KV_FP8", 32, 8, 64, 44, 128, True), ("KV_FP8", 32, 8, 64, 45, 128, False),
+    ("KV_FP8", 32, 8, 128, 16, 32, True), ("KV_FP8", 32, 8, 128, 16, 33, False),
+    ("KV_FP8", 64, 8, 64, 16, 32, True), ("KV_INT8", 32, 8, 64, 16, 64, True),
+    ("KV_INT8", 32, 8, 128, 16, 16, False), ("KV_INT8", 8, 2, 64, 16, 16, False)])
+def test_steps_of_few_rows_stay_on_the_decode_kernels(ehip_mod, monkeypatch, kv, H, Hkv, d, T, L,
+                                                      kept):
+    """A chunk without decode rows goes to the chunk kernel, but for few rows
+    over short contexts, which the decode kernels serve sooner in one launch;
+    EHIP_PREFILL=1 sends those too, EHIP_DECODE_WG=0 the fp32 ones."""
+    E = ehip_mod
+    g = geom(E, heads=H, kv_heads=Hkv, head_dim=d, kv_dtype=getattr(E, kv), slab_blocks=64)
+    st = simple_step(E, [L], qlens=np.array([T], np.int32))
+    assert (len(prefill_items(E, g, st)) == 0) == kept
+    monkeypatch.setenv("EHIP_DECODE_WG", "0")
+    assert (len(prefill_items(E, g, st)) == 0) == (kept and kv != "KV_F32")
+    monkeypatch.setenv("EHIP_PREFILL", "1")
+    assert len(prefill_items(E, g, st)) > 0
+
+
+@pytest.mark.parametrize("L,stays", [(769, True), (1024, True), (1025, False)])
+def test_few_rows_beside_a_decode_row_stay_longer(ehip_mod, L, stays):
+    """... by 256 keys, past the work that takes chunks off the decode kernels."""
+    E = ehip_mod
+    g = geom(E, heads=32, kv_heads=8, head_dim=64, kv_dtype=E.KV_F32, slab_blocks=96)
+    st = simple_step(E, [L, 40], qlens=np.array([31, 1], np.int32))
+    assert 31 * (L - 31) * 32 * 64 > 1 << 25
+    assert (len(prefill_items(E, g, st)) == 0) == stays
