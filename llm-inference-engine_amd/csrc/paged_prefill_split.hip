@@ -803,14 +803,31 @@ PrefillShape PrefillSplitShape(int kv_dtype, int d, int group, int64_t block_str
   s.slots = 256 * 8 / SplitWaves(kv_dtype);  // two wavefronts per SIMD
   s.min_tiles = 4;
   s.split = 1.0;
-  // Beside decode rows the chunks cost a launch of their own (~7 us a layer),
-  // which little work does not earn back. Four layers with 2 or 12 decode rows
-  // and 1 or 3 chunks of 16-204 rows, this kernel's time over the decode
-  // kernels', by pairs x heads x d: g = 4, fp32 1.05-1.38 at 21-24M and 0.58-0.71
-  // at 39-56M, FP8 1.05-1.21 and 0.82-0.95; g = 7, fp32 1.10 at 68M, 1.06 at 94M
-  // and 0.78-0.96 at 132-162M; g = 8, INT8 1.08-1.23 at 42-48M, 0.84-0.91 at
-  // 154-170M. Steps without decode rows: 0.2-1.0, whatever the work.
-  s.min_work = group > 4 ? int64_t{1} << 27 : int64_t{1} << 25;
+  // Beside decode rows the chunks cost a launch of their own (~6 us a layer),
+  // which little work does not earn back. Measured over 8,438 random steps (12
+  // layers; 1-64 decode rows, 1-3 chunks of 16-400 rows after 0-1500 keys; g 1
+  // to 8; steps of few rows apart), this kernel's time over the decode kernels',
+  // median (10th to 90th percentile), by pairs x kv heads x d, a kv head's heads
+  // sharing an item on the decode kernels:
+  //   fp32, g <= 4: 2-4M 1.26 (1.04-1.47), 4-9M 1.10 (0.71-1.44), 9-18M 0.87
+  //     (0.62-1.13), 18-36M 0.72; g > 4: 3-6M 1.11, 6-13M 1.03 (0.83-1.19),
+  //     13-26M 0.85 (0.69-1.03)
+  //   bf16, d = 64: g = 1 4-9M 1.13, 9-18M 1.04, 18-36M 0.86; g = 4 2-4M 1.21, 4-9M
+  //     0.96, 9-18M 0.85; g = 8 4-9M 1.09, 9-18M 1.00, 18-36M 0.84
+  //   INT8 and FP8: 5-9M 1.18 (1.07-1.33), 9-18M 1.10 (0.94-1.24), 18-36M 0.93
+  //     (0.77-1.12), 36-72M 0.77
+  // and by the chunk's context: past 130 keys its rows share 128 and more, which
+  // puts the whole decode launch on the joint items of two or four rows. At d =
+  // 128, g >= 4 that gives 0.46 (0.22-0.70) over fp32, 0.71 (0.42-0.94) over INT8
+  // and FP8 and 0.61 over bf16 whatever the work, 1.21 (1.06-1.34) up to there;
+  // bf16 at d = 64 0.62 to 0.75 (0.78 and 1.03 at g = 1 and 8). Outside bf16 the
+  // rule is within 15% of the faster side in 98 of 100 steps. The worst lose 1.24
+  // times (fp32, d = 64, g = 1, a 67-row chunk over 424 keys) where it takes this
+  // kernel and 1.66 (g = 4, three 110-row chunks) where it does not.
+  const bool scaled = kv_dtype != EHIP_KV_F32 && kv_dtype != EHIP_KV_BF16;
+  s.min_work = scaled ? 18'000'000 : group > 4 ? 13'000'000 : 10'000'000;
+  if (kv_dtype == EHIP_KV_BF16 ? d == 128 || (group != 1 && group != 8) : d == 128 && group >= 4)
+    s.any_work_keys = 130;
   SetFewRows(kv_dtype, d, group, &s);
   return s;
 }

@@ -626,16 +626,18 @@ int BuildPlan(const ehip_geometry& g, const ehip_step_desc& s, const Tuning& tun
   std::vector<int32_t> skip(plan->rows.size(), 0);
   bool chunk_kernel = prefill_rows > 0 && tune.prefill;
   if (chunk_kernel && shape.min_work > 0 && !tune.prefill_all) {
-    int64_t pairs = 0, units = 0;  // pairs below 2^24 rows x 2^31 keys
+    int64_t pairs = 0, units = 0, longest = 0;  // pairs below 2^24 rows x 2^31 keys
     bool decodes = false;
     for (int32_t b = 0; b < B; ++b) {
       const int64_t T = s.h_query_lens[b];
       const int64_t reads = T * (s.h_context_lens[b] - T) + T * (T + 1) / 2;
       units += reads * g.kv_heads;
-      if (T < shape.min_rows)
+      if (T < shape.min_rows) {
         decodes = true;
-      else
+      } else {
         pairs += reads;
+        longest = std::max(longest, s.h_context_lens[b]);
+      }
     }
     // Few rows, where the decode kernels write the outputs in one launch: fp32
     // on a workgroup per unit, INT8 and FP8 with one range a row.
@@ -645,10 +647,12 @@ int BuildPlan(const ehip_geometry& g, const ehip_step_desc& s, const Tuning& tun
             ? plan->max_length <= (units < kSmallStepUnits ? kTile : kMinSplit)
             : tune.decode_wg;
     if (one_launch && few >= shape.few_lo && few <= shape.few_hi &&
-        plan->max_length > shape.few_keys_lo &&
+        plan->max_length > shape.few_keys_lo && shape.few_keys_hi > 0 &&
         plan->max_length <= shape.few_keys_hi + (decodes ? kDecodesFewKeys : 0))
       chunk_kernel = false;
-    if (decodes && pairs < shape.min_work / (int64_t{g.heads} * g.head_dim)) chunk_kernel = false;
+    if (decodes && longest <= shape.any_work_keys &&
+        pairs < shape.min_work / (int64_t{g.kv_heads} * g.head_dim))
+      chunk_kernel = false;
   }
   if (chunk_kernel) {
     struct Block { int32_t b, q0, keys; };

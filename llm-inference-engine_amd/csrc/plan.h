@@ -211,9 +211,10 @@ int32_t SingleRowSplitTokens(const ehip_geometry& g, int64_t length, const Tunin
 // How the step's chunk kernel takes its work: query rows per item (0: no
 // kernel, chunk rows stay on the decode kernels), workgroups resident at once,
 // the least tiles of a key split, the shares of the step's tiles past which a
-// block is split, the shortest chunk, the work (attended pairs x heads x d of
+// block is split, the shortest chunk, the work (attended pairs x kv heads x d of
 // the step's chunks) below which a step with decode rows keeps its chunks on
-// their launch, and the steps of few rows that stay on the decode kernels: rows
+// their launch, unless one's context is past any_work_keys, and the steps of few
+// rows that stay on the decode kernels: rows
 // x kv heads in [few_lo, few_hi], longest context in (few_keys_lo, few_keys_hi].
 struct PrefillShape {
   int rows = 0;
@@ -222,6 +223,7 @@ struct PrefillShape {
   double split = 2.0;
   int32_t min_rows = 16;
   int64_t min_work = 0;
+  int32_t any_work_keys = INT32_MAX;
   int64_t few_lo = 0, few_hi = 0;
   int32_t few_keys_lo = 0, few_keys_hi = 0;
 };

@@ -608,17 +608,27 @@ def test_plan_every_row_keeps_a_range_ending_at_its_last_key(ehip_mod, L):
     assert joint[:, 5].max() <= (L - 1) // bs * bs
 
 
-@pytest.mark.parametrize("H,T,past", [(32, 16, 0), (32, 90, 0), (64, 170, 0), (64, 181, 0)])
-def test_small_chunks_beside_decode_rows_stay_with_them(ehip_mod, H, T, past):
-    """fp32 chunks leave a step's decode kernels from 2^25 attended pairs x
-    heads x d on (g = 4; 2^27 at g = 8), alone at any work."""
+@pytest.mark.parametrize("kv,H,d,T,past,moved", [
+    ("KV_F32", 32, 128, 16, 0, False), ("KV_F32", 32, 128, 90, 0, False),
+    ("KV_F32", 32, 128, 16, 114, False), ("KV_F32", 32, 128, 16, 115, True),
+    ("KV_F32", 64, 128, 170, 0, True), ("KV_F32", 16, 128, 138, 0, False),
+    ("KV_F32", 16, 128, 139, 0, False), ("KV_F32", 16, 128, 140, 0, True),
+    ("KV_F32", 64, 64, 224, 0, False), ("KV_F32", 64, 64, 225, 0, True),
+    ("KV_FP8", 32, 64, 264, 0, False), ("KV_FP8", 32, 64, 265, 0, True),
+    ("KV_FP8", 32, 128, 73, 57, False), ("KV_FP8", 32, 128, 73, 58, True),
+    ("KV_BF16", 8, 64, 100, 40, False), ("KV_BF16", 32, 64, 100, 40, True)])
+def test_small_chunks_beside_decode_rows_stay_with_them(ehip_mod, kv, H, d, T, past, moved):
+    """Chunks leave a step's decode kernels from 10M attended pairs x kv heads x
+    d on (fp32 and bf16 up to g = 4; 13M past it; 18M for INT8 and FP8), and
+    where they attend more than 130 keys at d = 128, g >= 4 (bf16: g = 2 and 4 at
+    d = 64 too). Alone they leave at any work."""
     E = ehip_mod
-    g = geom(E, heads=H, kv_heads=8, head_dim=128, kv_dtype=E.KV_F32, slab_blocks=64)
-    both = simple_step(E, [T + past, 40], qlens=np.array([T, 1], np.int32))
+    g = geom(E, heads=H, kv_heads=8, head_dim=d, kv_dtype=getattr(E, kv), slab_blocks=64)
+    both = simple_step(E, [T + past, 140], qlens=np.array([T, 1], np.int32))
     alone = simple_step(E, [T + past], qlens=np.array([T], np.int32))
-    work = T * (T + 1) // 2 * H * 128
-    assert (len(prefill_items(E, g, both)) > 0) == (work >= 1 << (27 if H == 64 else 25))
-    assert len(prefill_items(E, g, alone)) > 0
+    assert (len(prefill_items(E, g, both)) > 0) == moved
+    if H == 32 and d == 128 or T > 44:
+        assert len(prefill_items(E, g, alone)) > 0
 
 
 @pytest.mark.parametrize("kv,H,Hkv,d,T,L,kept", [
@@ -654,5 +664,5 @@ def test_few_rows_beside_a_decode_row_stay_longer(ehip_mod, L, stays):
     E = ehip_mod
     g = geom(E, heads=32, kv_heads=8, head_dim=64, kv_dtype=E.KV_F32, slab_blocks=96)
     st = simple_step(E, [L, 40], qlens=np.array([31, 1], np.int32))
-    assert 31 * (L - 31) * 32 * 64 > 1 << 25
+    assert 31 * (L - 31) * 8 * 64 > 10_000_000
     assert (len(prefill_items(E, g, st)) == 0) == stays
