@@ -35,6 +35,7 @@ def hip():
         h.hipGraphExecDestroy.argtypes = [vp]
         h.hipGraphDestroy.argtypes = [vp]
         h.hipGraphExecUpdate.argtypes = [vp, vp, C.POINTER(vp), C.POINTER(C.c_int)]
+        h.hipGraphGetNodes.argtypes = [vp, vp, C.POINTER(C.c_size_t)]
         _hip = h
     return _hip
 
@@ -42,6 +43,12 @@ def hip():
 def _ok(rc, what):
     if rc != 0:
         raise RuntimeError(f"{what} failed with hipError {rc}")
+
+
+def _nodes(graph) -> int:
+    n = C.c_size_t()
+    _ok(hip().hipGraphGetNodes(graph, None, C.byref(n)), "hipGraphGetNodes")
+    return n.value
 
 
 class Stream:
@@ -78,25 +85,41 @@ class Graph:
         return self
 
     def update(self, stream: Stream, fn):
-        """Re-capture what fn enqueues (the same launch sequence for a new step
-        plan) and write its kernel parameters into the instantiated graph
-        (hipGraphExecUpdate): no re-instantiation. Raises if the launch
-        topology changed (then capture() a new graph instead)."""
+        """Re-capture what fn enqueues for a new step plan and write its kernel
+        parameters into the instantiated graph (hipGraphExecUpdate). A plan with
+        other launches (chunks or split merges that come or go) replaces the
+        instantiated graph, once the stream has drained."""
         g = C.c_void_p()
         _ok(hip().hipStreamBeginCapture(stream.h, _CAPTURE_THREAD_LOCAL), "hipStreamBeginCapture")
         try:
             fn()
         finally:
             _ok(hip().hipStreamEndCapture(stream.h, C.byref(g)), "hipStreamEndCapture")
-        err_node, result = C.c_void_p(), C.c_int(-1)
-        rc = hip().hipGraphExecUpdate(self.exec, g, C.byref(err_node), C.byref(result))
-        if rc != 0:
+        try:
+            if not self._write(g):
+                new = C.c_void_p()
+                _ok(hip().hipGraphInstantiate(C.byref(new), g, None, None, 0),
+                    "hipGraphInstantiate")
+                stream.synchronize()
+                hip().hipGraphExecDestroy(self.exec)
+                self.exec = new
+        except RuntimeError:
             hip().hipGraphDestroy(g)
-            raise RuntimeError(f"hipGraphExecUpdate failed: hipError {rc}, update result "
-                               f"{result.value}")
+            raise
         hip().hipGraphDestroy(self.graph)
         self.graph = g
         return self
+
+    def _write(self, g) -> bool:
+        """g's parameters into the instantiated graph; False if its launches
+        are others."""
+        if _nodes(g) != _nodes(self.graph):
+            return False
+        err_node, result = C.c_void_p(), C.c_int(-1)
+        if hip().hipGraphExecUpdate(self.exec, g, C.byref(err_node), C.byref(result)) == 0:
+            return True
+        hip().hipGetLastError()  # the refusal is no error of the next launch
+        return False
 
     def replay(self, stream: Stream):
         _ok(hip().hipGraphLaunch(self.exec, stream.h), "hipGraphLaunch")

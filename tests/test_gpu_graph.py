@@ -245,3 +245,69 @@ def test_graph_replay_follows_a_changing_decode_plan(gctx, ehip_mod, orc):
         gs.close()
     for x in [b for pair in dev for b in pair] + [b for s in drows for l in s for b in l] + outs:
         x.free()
+
+
+@pytest.mark.parametrize("fmt", ["f32", "fp8"])
+def test_graph_follows_chunks_that_come_and_go(gctx, ehip_mod, orc, fmt):
+    """One graph over steps whose launches differ: decode rows alone, with a
+    chunk below and above the work that takes it to the chunk kernel, a chunk
+    alone (whole, then in key splits), decode rows again. Every replay is bit-identical to the eager run."""
+    from ehip import hipgraph
+    E = ehip_mod
+    H, Hkv, d, bs = 32, 8, 128, 16
+    fp8 = fmt == "fp8"
+    steps = [([1] * 6, [300, 60, 700, 17, 513, 90]),
+             ([1, 1, 24], [301, 61, 24]), ([1, 1, 230], [302, 62, 230]),
+             ([70], [100]), ([60], [700]), ([1] * 6, [303, 63, 701, 18, 514, 91])]
+    pool = 200
+    rng = np.random.default_rng(21)
+    shape = (pool, Hkv, bs, d)
+    if fp8:
+        slabs = [rng.integers(0, 0x70, shape).astype(np.uint8) for _ in "kv"]
+        scales = [rng.uniform(0.002, 0.006, (pool, Hkv)).astype(np.float32) for _ in "kv"]
+    else:
+        slabs, scales = [rng.standard_normal(shape).astype(np.float32) for _ in "kv"], []
+    dev = [gctx.to_device(x) for x in slabs + scales]
+    g = E.geometry(H, Hkv, d, bs, E.KV_FP8 if fp8 else E.KV_F32, pool, 1 / np.sqrt(d))
+    gs, graph = hipgraph.Stream(), hipgraph.Graph()
+    assert E.lib().ehip_set_stream(gctx.h, gs.h) == 0
+    bufs = []
+    try:
+        for qlens, lens in steps:
+            perm = rng.permutation(pool).astype(np.int32)
+            need = np.cumsum([0] + [-(-n // bs) for n in lens])
+            tabs = [perm[a:b] for a, b in zip(need[:-1], need[1:])]
+            slots = np.concatenate([[int(t[p // bs]) * bs + p % bs for p in range(n - q, n)]
+                                    for t, q, n in zip(tabs, qlens, lens)]).astype(np.int64)
+            R = sum(qlens)
+            kn, vn = (rng.standard_normal((R, Hkv, d)).astype(np.float32) for _ in "kv")
+            q = rng.standard_normal((R, H, d)).astype(np.float32)
+            dkn, dvn, dq = (gctx.to_device(x) for x in (kn, vn, q))
+            out = gctx.alloc(q.nbytes)
+            bufs += [dkn, dvn, dq, out]
+
+            def launches():
+                sfx = "_fp8" if fp8 else ""
+                assert getattr(gctx, "step_kv_append" + sfx)(dkn, dvn, *dev) == 0
+                assert getattr(gctx, "step_attention" + sfx)(dq, *dev, out) == 0
+
+            assert gctx.step_upload(g, E.StepArrays(qlens, lens, tabs, slots)) == 0
+            launches()
+            gctx.sync()
+            eager = out.download(np.float32, q.shape).copy()
+            if graph.exec:
+                graph.update(gs, launches)
+            else:
+                graph.capture(gs, launches)
+            for _ in range(3):  # the append writes the same rows again
+                out.upload(np.full(q.shape, -7.0, np.float32))
+                graph.replay(gs)
+                gctx.sync()
+                got = out.download(np.float32, q.shape)
+                assert np.array_equal(got.view(np.uint32), eager.view(np.uint32)), (qlens, lens)
+    finally:
+        assert E.lib().ehip_set_stream(gctx.h, None) == 0
+        graph.close()
+        gs.close()
+    for b in bufs + dev:
+        b.free()
