@@ -48,6 +48,14 @@ constexpr int32_t kDecodesFewKeys = 256;
 constexpr int64_t kLargeStep = 512;
 constexpr int64_t kLargeMin = 1024;
 constexpr int64_t kLargeMax = 1536;
+// INT8/FP8 steps at d = 128 and g <= 4 whose ranges would be longer than
+// kScaledLong keys take kScaledMax: their last items' walks weigh less than the
+// startups. us a layer at ranges of the target's length / 2048 keys, INT8, 8 kv
+// heads: g = 1 132.6/137.8 at 1292, 147.2/143.5 at 1449, 170.6/165.7 at 1698,
+// 197.4/195.7 at 1984; g = 4 140.7/149.9, 155.7/156.5, 181.3/176.7, 208.0/204.9.
+// Not at g = 8 (200.8/204.6 at 1698) or d = 64 (107.6/109.9).
+constexpr int64_t kScaledLong = 1400;
+constexpr int64_t kScaledMax = 2048;
 
 int Fail(std::string* err, int code, const char* fmt, long long a = 0, long long b = 0,
          long long c = 0) {
@@ -177,6 +185,9 @@ int32_t ChooseSplitTokens(const ehip_geometry& g, int64_t unit_tokens, const Tun
   const int64_t target = DecodeItemTarget(tune);
   int64_t s = (unit_tokens + target - 1) / target;
   if (!ScaledKv(g.kv_dtype) && s >= kLargeStep) s = std::clamp(s, kLargeMin, kLargeMax);
+  if (ScaledKv(g.kv_dtype) && g.head_dim == 128 && g.heads / g.kv_heads <= 4 &&
+      s > kScaledLong && s < kScaledMax)
+    s = kScaledMax;
   s = RoundUp(std::max<int64_t>(s, unit_tokens < kSmallStepUnits ? kTile : kMinSplit), kTile);
   return static_cast<int32_t>(std::min<int64_t>(s, max_split));
 }

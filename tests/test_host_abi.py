@@ -171,7 +171,7 @@ def test_plan_large_steps_take_1024_to_1536_key_ranges(ehip_mod):
         rc, rows, items, partials, split = ehip_mod.plan_counts(
             geom(ehip_mod, slab_blocks=256 * ((L + 15) // 16)), simple_step(ehip_mod, lens))
         assert rc == 0 and split == want, (L, split)
-    # INT8 keeps its own rule (half the item target, 128-block ranges).
+    # INT8 keeps its own length cap (128-block ranges).
     w = workloads.c4()
     g = ehip_mod.geometry(w.heads, w.kv_heads, w.head_dim, w.block_size, ehip_mod.KV_INT8,
                           w.pool_blocks, w.scale)
@@ -666,3 +666,16 @@ def test_few_rows_beside_a_decode_row_stay_longer(ehip_mod, L, stays):
     st = simple_step(E, [L, 40], qlens=np.array([31, 1], np.int32))
     assert 31 * (L - 31) * 8 * 64 > 10_000_000
     assert (len(prefill_items(E, g, st)) == 0) == stays
+
+
+@pytest.mark.parametrize("kv", ["KV_INT8", "KV_FP8"])
+@pytest.mark.parametrize("H,Hkv,d,keys,want", [
+    (32, 8, 128, 1400, 1408), (32, 8, 128, 1401, 2048), (8, 8, 128, 1900, 2048),
+    (32, 8, 128, 2100, 2048), (64, 8, 128, 1500, 1536), (32, 8, 64, 1500, 1536)])
+def test_scaled_ranges_past_1400_keys_take_2048(ehip_mod, kv, H, Hkv, d, keys, want):
+    """256 rows of one range each at the item target's length (`keys`)."""
+    E = ehip_mod
+    blocks = (keys + 15) // 16
+    g = geom(E, heads=H, kv_heads=Hkv, head_dim=d, kv_dtype=getattr(E, kv),
+             slab_blocks=256 * blocks)
+    assert E.plan_counts(g, simple_step(E, [keys] * 256))[4] == want
