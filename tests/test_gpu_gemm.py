@@ -103,7 +103,9 @@ def test_wide_tiles_at_their_edges(gctx, ehip_mod, orc, m, k, n):
     """bf16 weights with k % 32 == 0 (tiles of 16-128 rows x 256 columns): row
     and column remainders, odd step counts, k splits of the last round's tiles
     (the last shape has one whole round of them), and x and y 4 bytes off a
-    16-byte boundary. Bar: the reference's GEMM tolerance, against 64 bits."""
+    16-byte boundary. Bars, against 64 bits: the reference's GEMM tolerance, and
+    1e-6 in the 2-norm, what fp32 sums of up to 4096 terms in groups give
+    (6.5e-7 there; x in two planes: about 1.5e-6)."""
     x = orc.fill_normal(m * k, 0.0, 1.0, m + k).reshape(m, k)
     w = _weights(orc, ehip_mod, n, k, ehip_mod.WEIGHT_BF16, n + k)
     bias = orc.fill_normal(n, 0.0, 1.0, 9)
@@ -123,8 +125,37 @@ def test_wide_tiles_at_their_edges(gctx, ehip_mod, orc, m, k, n):
     err = np.abs(out[1:-1].reshape(m, n) - ref)
     bad = err > 1e-5 * np.sqrt(k) + 1e-4 * np.abs(ref)
     assert not bad.any(), (int(bad.sum()), float(err.max()))
+    assert np.linalg.norm(err) <= 1e-6 * np.linalg.norm(ref)
     for b in (dw, db, dwp, dx, dy):
         b.free()
+
+
+@pytest.mark.parametrize("m,k,n", [(16, 64, 256), (32, 896, 896), (130, 4096, 512),
+                                   (2100, 64, 4096)])
+@pytest.mark.parametrize("wt", ["WEIGHT_BF16", "WEIGHT_F16", "WEIGHT_F32"])
+def test_third_plane_of_x_reaches_y(gctx, ehip_mod, orc, wt, m, k, n):
+    """x = 1 + 1.5 * 2^-9 + b * 2^-18 with b in -1, 0, 1: its bf16 planes are 1,
+    1.5 * 2^-9 and b * 2^-18. Weights come in pairs (w, -w), w = +-1, so that
+    y = 2^-18 sum(b w): only the third plane is left. Every partial sum of a
+    step is exact in fp32 (from 2^5 down to 2^-18), so y is to a quarter unit."""
+    rng = np.random.default_rng(m + k)
+    b = rng.integers(-1, 2, (m, k))
+    x = (1 + 1.5 * 2.0**-9 + b * 2.0**-18).astype(np.float32)
+    assert np.array_equal(x.astype(np.float64), 1 + 1.5 * 2.0**-9 + b * 2.0**-18)
+    w = np.repeat(rng.choice([-1, 1], (n, k // 2)), 2, axis=1)
+    w[:, 1::2] *= -1
+    dtype = getattr(ehip_mod, wt)
+    raw = {"WEIGHT_F32": w.astype(np.float32), "WEIGHT_F16": w.astype(np.float16).view(np.uint16),
+           "WEIGHT_BF16": (w.astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)}[wt]
+    dx, dw = gctx.to_device(x), gctx.to_device(raw)
+    dwp, dy = gctx.alloc(((n + 15) // 16) * k * 16 * raw.itemsize), gctx.alloc(4 * m * n)
+    assert gctx.pack_weight_panels(dw, dtype, n, k, dwp) == 0
+    assert gctx.packed_gemm(dx, m, k, dwp, dtype, n, None, dy) == 0
+    gctx.sync()
+    got = dy.download(np.float32, (m, n)).astype(np.float64) * 2.0**18
+    assert np.abs(got - b.astype(np.float64) @ w.T.astype(np.float64)).max() <= 0.25
+    for buf in (dx, dw, dwp, dy):
+        buf.free()
 
 
 def test_packed_gemm_validates(gctx, ehip_mod):

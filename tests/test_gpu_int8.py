@@ -276,3 +276,44 @@ def test_scaled_chunks_match_the_decode_kernels(ehip_mod, orc, tctx, fmt, H, Hkv
         outs.append(got)
         run.free()
     assert rel_norm(outs[0], outs[1]) <= 1e-4
+
+
+@pytest.mark.parametrize("fmt", FORMATS)
+@pytest.mark.parametrize("d,T", [(128, 1), (128, 16), (64, 40)])
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_append_of_non_finite_rows(gctx, ehip_mod, orc, fmt, d, T, bad):
+    """A NaN takes no part in its block's maximum and becomes code 0x7F (E4M3)
+    or -127 (INT8); an infinity makes the block's scale infinite, its own code
+    that of NaN (inf * 0) and the others 0. Blocks, heads and K/V without one
+    are bit-identical to the oracle's."""
+    E, Hkv, bs = ehip_mod, 2, 16
+    nb = (T + 15) // 16 + 1
+    rng = np.random.default_rng(d + T)
+    kn, vn = (rng.standard_normal((T, Hkv, d)).astype(np.float32) for _ in "kv")
+    k, v = (np.zeros((nb, Hkv, bs, d), np.uint8 if fmt == "fp8" else np.int8) for _ in "kv")
+    ks, vs = np.ones((nb, Hkv), np.float32), np.ones((nb, Hkv), np.float32)
+    slots = np.arange(T, dtype=np.int64)
+    row, col = T - 1, 5
+    kn[row, 1, col] = 0.0
+    dev = [gctx.to_device(x) for x in (kn, vn, k, v, ks, vs)]
+    bad_kn = kn.copy()
+    bad_kn[row, 1, col] = bad
+    dev[0].upload(bad_kn)
+    getattr(orc, f"kv_append_{fmt}")(kn, vn, slots, Hkv, d, bs, k, v, ks, vs)
+    blk, off = divmod(row, bs)
+    if np.isinf(bad):
+        k[blk, 1, :off + 1] = 0
+        if fmt == "fp8":
+            k[blk, 1, :off + 1] = np.signbit(kn[blk * bs:, 1]) * 0x80
+        ks[blk, 1] = np.inf
+    k[blk, 1, off, col] = 0x7F if fmt == "fp8" else -127
+    g = E.geometry(4, Hkv, d, bs, E.KV_FP8 if fmt == "fp8" else E.KV_INT8, nb, 1.0)
+    st = E.StepArrays([T], [T], [np.arange(nb, dtype=np.int32)], slots)
+    assert gctx.step_upload(g, st) == 0, gctx.last_error()
+    assert getattr(gctx, f"step_kv_append_{fmt}")(*dev) == 0, gctx.last_error()
+    gctx.sync()
+    for b, want in zip(dev[2:], (k, v, ks, vs)):
+        assert np.array_equal(b.download(want.dtype, want.shape).view(np.uint8),
+                              want.view(np.uint8))
+    for b in dev:
+        b.free()
