@@ -215,7 +215,7 @@ struct GemmParams {
   int64_t k_split;      // k per split (a multiple of 32)
   int32_t splits;
   int32_t x_vec;        // x rows are 16-byte aligned (k % 4 == 0, aligned base)
-  // The wide kernel (bf16 weights, k % 32 == 0): tiles of tile_rows x 256, the
+  // The wide kernel (bf16 weights, k % 32 == 0; see PlanWide): tiles of tile_rows x 256, the
   // first full_tiles whole, the others in `splits` k ranges of split_steps
   // 32-k steps; tile_rows = 0: the other kernel.
   int32_t tile_rows;

@@ -7,8 +7,8 @@
 // accumulation, and the bias added once after the k sum
 // (src/kernels/internal/gemm_common.h:22-41).
 //
-// Two kernels: PackedGemmWide for bf16 weights with k % 32 == 0 (below), and
-// PackedGemmMfma for the rest.
+// Two kernels: PackedGemmWide for bf16 weights with k % 32 == 0 (below, but for
+// short sums of many rows), and PackedGemmMfma for the rest.
 //
 // Matrix-core form: every operand is cut into bf16 planes whose sum is the
 // value. x (fp32) takes three (x = x0 + x1 + x2, each the RNE bf16 of what the
@@ -608,7 +608,8 @@ __global__ __launch_bounds__(256) void PackPanels(const T* w, int64_t n, int64_t
 namespace {
 
 // Row tile of the wide kernel for m rows: the one whose padded rows, with 32
-// rows' worth of panel staging per tile, come out smallest.
+// rows' worth of panel staging per tile, come out smallest. The partial sums of
+// a split last round, whose bytes grow with the tile's rows, are not counted.
 int WideRows(int64_t m) {
   int best = 128;
   int64_t cost = INT64_MAX;
@@ -624,6 +625,12 @@ int WideRows(int64_t m) {
 
 bool PlanWide(int64_t m, int64_t k, int64_t n, int cus, GemmParams* p) {
   if (k % kWideK != 0 || k > (int64_t{1} << 21)) return false;  // whole steps, 32-bit offsets
+  // Short sums of many rows are over before this kernel's loads are two steps
+  // ahead. The other kernel / this one, us a call at n = 256 (4096): k = 64 10.4/
+  // 12.8 (10.8/13.5) at 300 rows, 10.8/13.1 (22/26) at 2382; k = 192 13.4/16.7
+  // (14.1/17.4) at 300; k = 256 14.0/11.1 (22.5/17.3). Up to 256 rows, where the
+  // other one has 256-column tiles, 14.5/12.8 at k = 64 and 200 rows.
+  if (k < 256 && m > 256) return false;
   const int tm = WideRows(m);
   const int64_t rt = (m + tm - 1) / tm, ct = (p->panels + 15) / 16;
   if (rt * ct > (int64_t{1} << 24)) return false;
@@ -656,17 +663,17 @@ bool PlanWide(int64_t m, int64_t k, int64_t n, int cus, GemmParams* p) {
 }  // namespace
 
 void PlanPackedGemm(int64_t m, int64_t k, int64_t n, int weight_dtype, int cus, GemmParams* p) {
-  // 16 panels (256 columns) per workgroup for bf16 weights and up to 256
-  // rows: each x row is then staged for twice the columns (C4 o_proj 58.5 ->
-  // 56 us, C5 63 -> 60 us). Taller calls keep 8 (C3's 2382 rows: 350 against
-  // 365 us at 16), as do fp16 and fp32 weights, whose two or three weight
-  // planes would not fit LDS at 16.
   p->m = m;
   p->k = k;
   p->n = n;
   p->panels = (n + kNr - 1) / kNr;
   p->tile_rows = 0;
   if (weight_dtype == EHIP_WEIGHT_BF16 && PlanWide(m, k, n, cus, p)) return;
+  // 16 panels (256 columns) per workgroup for bf16 weights and up to 256 rows:
+  // each x row is then staged for twice the columns (58.5 -> 56 us at 256 x 4096
+  // x 4096, 365 against 350 us at 2382 rows, measured before the wide kernel took
+  // whole 32-k steps). fp16 and fp32 weights keep 8: their two or three planes
+  // would not fit LDS at 16.
   const int kBP = (weight_dtype == EHIP_WEIGHT_BF16 && m <= 256) ? 16 : 8;
   p->group_panels = kBP;
   p->m_pad = (m + kBM - 1) / kBM * kBM;

@@ -98,11 +98,12 @@ def test_packed_gemm_split_k_is_deterministic(gctx, ehip_mod, orc):
 @pytest.mark.parametrize("m,k,n", [
     (1, 32, 16), (16, 96, 250), (17, 64, 256), (31, 128, 257), (33, 4096, 1111), (64, 160, 896),
     (65, 896, 896), (127, 64, 4112), (128, 544, 272), (129, 256, 512), (257, 2048, 1000),
-    (2100, 64, 4096)])
+    (2100, 64, 4096), (2100, 256, 4096), (300, 224, 512), (256, 224, 512), (257, 256, 250)])
 def test_wide_tiles_at_their_edges(gctx, ehip_mod, orc, m, k, n):
     """bf16 weights with k % 32 == 0 (tiles of 16-128 rows x 256 columns): row
     and column remainders, odd step counts, k splits of the last round's tiles
-    (the last shape has one whole round of them), and x and y 4 bytes off a
+    (2100 rows have one whole round of them), both sides of the line where short
+    sums of many rows leave them (k < 256, m > 256), and x and y 4 bytes off a
     16-byte boundary. Bars, against 64 bits: the reference's GEMM tolerance, and
     1e-6 in the 2-norm, what fp32 sums of up to 4096 terms in groups give
     (6.5e-7 there; x in two planes: about 1.5e-6)."""
