@@ -37,13 +37,15 @@
  *     left out is below 2^-24 of |q||k| per element), and is all-fp32 on the
  *     vector ALUs at other head sizes; INT8 KV forms exact integer q.k
  *     products of a three-digit int8 split of q; FP8 KV widens the E4M3 keys
- *     to bf16 (exact) and multiplies them by q in bf16 hi + lo parts. Causal
- *     prefill chunks over bf16 K/V with d = 128, g 4 or 8 and bs >= 16 round q
- *     and the probabilities P to bf16 for their matrix-core products (fp32
- *     accumulate); every other chunk at d 64 or 128 multiplies bf16 planes
- *     that sum to the operands (three of q, two over FP8 K/V; three of P;
- *     K/V exact), which keeps the decode kernels' precision. The parity bars
- *     these give are stated beside each test.
+ *     to bf16 (exact) and multiplies them by q in bf16 hi + lo parts (up to
+ *     2^-18 of q left out). Causal prefill chunks over bf16 K/V with d = 128,
+ *     g 4 or 8, bs >= 16 and slabs below 4 GiB round q and the probabilities P
+ *     to bf16 for their matrix-core products (fp32 accumulate); the other
+ *     chunks at d 64 or 128 that leave the decode kernels multiply bf16 planes
+ *     of the operands (three of q and of P, whose sums are the operands to
+ *     2^-24; two of q over FP8 K/V, as in its decode; K/V exact), which keeps
+ *     the decode kernels' precision. The parity bars these give are stated
+ *     beside each test.
  *   - A context is used from one host thread at a time (the reference's
  *     single engine thread, src/runtime/engine.h:27-33).
  */

@@ -13,8 +13,8 @@
 // first. fp32 K and V take three planes, int8, E4M3 and bf16 values are one
 // plane exactly; q takes three (two over FP8 K/V, the split its decode kernel
 // uses), the probabilities three. What is left out is below 2^-24 of the
-// factors' magnitudes, so a row agrees with the decode kernels' fp32-class
-// result. Scales multiply the finished scores (K) and the probabilities (V).
+// factors' magnitudes (over FP8 K/V below 2^-18, q's third plane), so a row
+// agrees with the decode kernels' result. Scales multiply the finished scores (K) and the probabilities (V).
 //
 // Work: one workgroup of 4 wavefronts (8 over fp32 K/V) per (chunk, kv head,
 // up to 64 or 128 query vectors). A vector is one (row, query head) pair; a kv
@@ -151,8 +151,8 @@ __device__ __forceinline__ void SplitPair(float x, float y, PairFactors f, uint3
 // Bits of |v| from which the RNE bf16 is not finite.
 constexpr uint32_t kBf16Overflow = 0x7F7F8000u;
 
-template <int KV, int D, int WAVES, int HB, int NBUF, int OCC>
-__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC)))
+template <int KV, int D, int WAVES, int HB>
+__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2)))
 void PrefillSplitMfma(PrefillParams p) {
   constexpr int kThreads = WAVES * 64;
   using KT = KvTraits<KV>;
@@ -169,9 +169,9 @@ void PrefillSplitMfma(PrefillParams p) {
   constexpr int NID = NV > 1 ? NV / 2 : 1;        // distinct rows per thread
   static_assert(NV >= 1 && NV * kThreads == 2 * kTile * VPR, "tile / block shape");
 
-  __shared__ __align__(16) unsigned char tiles[NBUF][2 * KP * PLANE];
-  __shared__ __align__(16) float tile_scale[NBUF][4];  // K, V scales of the tile's halves
-  __shared__ __align__(16) int tile_odd[NBUF][WAVES];  // non-finite V (1), K (2) a wavefront saw
+  __shared__ __align__(16) unsigned char tiles[2][2 * KP * PLANE];
+  __shared__ __align__(16) float tile_scale[2][4];  // K, V scales of the tile's halves
+  __shared__ __align__(16) int tile_odd[2][WAVES];  // non-finite V (1), K (2) a wavefront saw
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -695,8 +695,7 @@ void PrefillSplitMfma(PrefillParams p) {
   }
 #define EHIP_PS_STEP(T, ST, IDC, IDN)                            \
   do {                                                           \
-    const int buf = NBUF == 2 ? ((T) & 1) : 0;                    \
-    if constexpr (NBUF == 1) EHIP_PS_BARRIER();                   \
+    const int buf = (T) & 1;                                      \
     store_tile(ST, buf);                                          \
     EHIP_PS_FENCE();                                              \
     load_ids(key0 + ((T) + 3) * kTile, IDN);                      \
@@ -839,22 +838,21 @@ bool LaunchPrefillSplit(const PrefillParams& p, int kv_dtype, hipStream_t stream
     return true;
   }
   const dim3 grid(p.n_items);
-#define EHIP_PREFILL_SPLIT_CASE(KK, DD, NBUF, OCC)                                            \
+#define EHIP_PREFILL_SPLIT_CASE(KK, DD)                                                       \
   if (kv_dtype == KK && p.d == DD) {                                                          \
-    hipLaunchKernelGGL(                                                                       \
-        (PrefillSplitMfma<KK, DD, SplitWaves(KK), SplitBlocks(KK, DD), NBUF, OCC>), grid, \
-        dim3(SplitWaves(KK) * 64), 0, stream, p);                                         \
+    hipLaunchKernelGGL((PrefillSplitMfma<KK, DD, SplitWaves(KK), SplitBlocks(KK, DD)>), grid, \
+                       dim3(SplitWaves(KK) * 64), 0, stream, p);                              \
     *err = hipGetLastError();                                                                 \
     return true;                                                                              \
   }
-  EHIP_PREFILL_SPLIT_CASE(EHIP_KV_F32, 64, 2, 2)
-  EHIP_PREFILL_SPLIT_CASE(EHIP_KV_F32, 128, 2, 2)
-  EHIP_PREFILL_SPLIT_CASE(EHIP_KV_BF16, 64, 2, 2)
-  EHIP_PREFILL_SPLIT_CASE(EHIP_KV_BF16, 128, 2, 2)
-  EHIP_PREFILL_SPLIT_CASE(EHIP_KV_INT8, 64, 2, 2)
-  EHIP_PREFILL_SPLIT_CASE(EHIP_KV_INT8, 128, 2, 2)
-  EHIP_PREFILL_SPLIT_CASE(EHIP_KV_FP8, 64, 2, 2)
-  EHIP_PREFILL_SPLIT_CASE(EHIP_KV_FP8, 128, 2, 2)
+  EHIP_PREFILL_SPLIT_CASE(EHIP_KV_F32, 64)
+  EHIP_PREFILL_SPLIT_CASE(EHIP_KV_F32, 128)
+  EHIP_PREFILL_SPLIT_CASE(EHIP_KV_BF16, 64)
+  EHIP_PREFILL_SPLIT_CASE(EHIP_KV_BF16, 128)
+  EHIP_PREFILL_SPLIT_CASE(EHIP_KV_INT8, 64)
+  EHIP_PREFILL_SPLIT_CASE(EHIP_KV_INT8, 128)
+  EHIP_PREFILL_SPLIT_CASE(EHIP_KV_FP8, 64)
+  EHIP_PREFILL_SPLIT_CASE(EHIP_KV_FP8, 128)
 #undef EHIP_PREFILL_SPLIT_CASE
   return false;
 }

@@ -43,7 +43,7 @@ struct Tuning {
                                // always / never (default: when items <= the item target)
   bool joint = true;           // EHIP_NO_JOINT=1: no joint items over shared prefixes
   bool prefill = true;         // EHIP_PREFILL=0: chunk rows stay on the decode kernels
-  bool prefill_all = false;    // EHIP_PREFILL=1: small chunks beside decode rows leave them too
+  bool prefill_all = false;    // EHIP_PREFILL=1: every chunk leaves the decode kernels
   double prefill_split = -1;   // EHIP_PREFILL_SPLIT: key-split threshold in shares (0: none;
                                // default: the chunk kernel's own, PrefillShape)
   int32_t prefill_tiles = 0;   // EHIP_PREFILL_TILES: least tiles of a key split (0: the kernel's)
