@@ -304,7 +304,7 @@ __global__ __launch_bounds__(kThreads) void PackedGemmMfma(GemmParams p) {
 // read; panel rows sit as stored and are read transposed.
 //
 // Bound by the matrix cores' issue with two wavefronts a SIMD in step (MFMA busy
-// ~50% of a long call). Measured, this kernel against the other: 2382 x 4096 x
+// 56% of a 2382-row call, 32% at 256 rows). Measured, this kernel against the other: 2382 x 4096 x
 // 4096 200 against 291 us a call, 256 x 4096 x 4096 35 against 51 us (28.6 + 7.4
 // us of split reduce), 32 x 896 x 896 9.3 against 21 us, 32 x 8192 x 8192 42
 // against 53 us. Interleaving the cuts with the MFMAs by scheduling groups took
