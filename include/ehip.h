@@ -260,10 +260,10 @@ int ehip_packed_gemm(ehip_ctx* ctx, const float* d_x, int64_t m, int64_t k, cons
  * L_b = h_l_dims[b] >= T_b: P_b = L_b - T_b cached keys, then the chunk's).
  * cu_seqlens, the pointer arrays and l_dims are host arrays (the K/V they
  * point at are device memory). Every sequence is validated before anything is
- * launched; then all of them run in one plan and launch of the chunk kernel
- * (d 64 or 128; the split merge follows), or at other head sizes one by one
- * through the paged kernels, as ehip_prefill_attention_f32. num_seqs == 0 is a
- * no-op. fp32. */
+ * launched; then two and more run in one plan and launch of the chunk kernel
+ * (d 64 or 128; the split merge follows), a single one, or each at other head
+ * sizes, through the paged kernels, as ehip_prefill_attention_f32. num_seqs == 0
+ * is a no-op. fp32. */
 int ehip_prefill_attention_varlen_f32(ehip_ctx* ctx, const float* d_q,
                                       const int32_t* h_cu_seqlens, int64_t num_seqs,
                                       const float* const* h_k_seqs,
